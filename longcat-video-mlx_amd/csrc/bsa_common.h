@@ -194,6 +194,11 @@ struct AttnParams {
 // Chooses the MFMA kernel (fp16/bf16, D in {64,128}, scale >= 0) or the
 // vector-ALU kernel (any dtype, D in {16,32,64,128,256}).
 hipError_t launch_attn(const AttnParams& p, int dtype, int D, hipStream_t stream);
+// fp32 inputs on split-bf16 MFMAs: D in {64, 128}, rows of 16-byte aligned
+// float4s and heads of k / v below 4 GiB (attn_f32_usable); other fp32 inputs
+// take the vector-ALU kernel.
+bool attn_f32_usable(const AttnParams& p, int D);
+hipError_t launch_attn_f32(const AttnParams& p, int D, hipStream_t stream);
 bool attn_supported(int dtype, int D);
 bool attn_uses_mfma(int dtype, int D);
 
