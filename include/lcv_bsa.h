@@ -375,6 +375,41 @@ int lcv_bsa_prepare_qk(const void* q_in, const void* k_in, int dtype,
                        lcv_bsa_strides k_out_strides, float* qbar, float* kbar,
                        void* stream);
 
+/*
+ * lcv_bsa_prepare_qk where k (and v) continue a cache of S_cache earlier
+ * tokens: the KV-cache continuation of the attention layer
+ * (longcat_video/models/attention.py:235-275: norms, torch.cat of cache and new
+ * k / v, q zero-padded to align its positions, rope_3d over the whole grid) in
+ * one pass, and, with S_cache = 0, the pass that fills such a cache
+ * (attention.py:191-201, which keeps k after its norm and before RoPE).
+ *   q_out  [B,H,Sq,D]          RMSNorm and RoPE at positions S_cache ..;
+ *   k_out  [B,H,S_cache+Sq,D]  RoPE of the cached rows (already normed), then
+ *                              RMSNorm and RoPE of the new rows;
+ *   v_out  [B,H,S_cache+Sq,D]  cached, then new rows; v_in, v_cache and v_out
+ *                              are given together, or all NULL;
+ *   k_norm [B,H,Sq,D]          the new k rows after RMSNorm, or NULL;
+ *   qbar / kbar                block means of q_out (geometry gq) and k_out (gk).
+ * k_cache is given when S_cache > 0; a batch stride of 0 shares one cache.
+ * rope is the grid of all S_cache + Sq tokens.  Dtypes, head dims, blocks and
+ * alignment as lcv_bsa_prepare_qk.
+ */
+int lcv_bsa_prepare_qkv(const void* q_in, const void* k_in, const void* v_in,
+                        int dtype, int64_t B, int64_t H, int64_t Sq, int64_t D,
+                        lcv_bsa_strides q_in_strides, lcv_bsa_strides k_in_strides,
+                        lcv_bsa_strides v_in_strides, const void* k_cache,
+                        const void* v_cache, int64_t S_cache,
+                        lcv_bsa_strides k_cache_strides,
+                        lcv_bsa_strides v_cache_strides, const void* q_weight,
+                        const void* k_weight, float eps, lcv_bsa_grid rope,
+                        const float* rope_table, int64_t rope_table_len,
+                        lcv_bsa_geom gq, lcv_bsa_geom gk, void* q_out,
+                        void* k_out, void* v_out, void* k_norm,
+                        lcv_bsa_strides q_out_strides,
+                        lcv_bsa_strides k_out_strides,
+                        lcv_bsa_strides v_out_strides,
+                        lcv_bsa_strides k_norm_strides, float* qbar,
+                        float* kbar, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

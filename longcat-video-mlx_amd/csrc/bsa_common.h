@@ -221,6 +221,21 @@ hipError_t launch_prep(const Tensor4* in, const Tensor4* out, const void* const*
                        const int32_t* rope_grid, const int32_t* rope_dims, const float* table,
                        int table_len, float eps, hipStream_t stream);
 
+// The same where k (and v) continue a cache: k_cache holds `cached` normed,
+// un-rotated rows; out k / v hold cached + new rows in geometry gk (nk blocks).
+// v_out.ptr null: v is not gathered.  k_norm.ptr, if set, receives the new k
+// rows after the norm.
+struct PrepCached {
+  Tensor4 in[2], out[2];  // q, new k; q, whole k
+  const void* weight[2];
+  float* mean[2];
+  Tensor4 v_in, v_out, k_cache, v_cache, k_norm;
+  int cached;
+};
+hipError_t launch_prep_cached(const PrepCached& x, int dtype, int B, int H, int D, int nb, int nk, const Geom& g,
+                              const Geom& gk, const int32_t* rope_grid, const int32_t* rope_dims, const float* table,
+                              int table_len, float eps, hipStream_t stream);
+
 // DiT block row operations (fp16 / bf16).
 bool rows_supported(int dtype, int C);
 hipError_t launch_rows(const void* x, const void* a, const float* gate, const float* shift,

@@ -731,6 +731,48 @@ int64_t lcv_bsa_rope_table_len(int64_t D, lcv_bsa_grid rope) {
   return len <= lcv::kMaxRopeTable ? len : 0;
 }
 
+}  // extern "C"
+
+namespace {
+
+// RoPE grid, table and weights of the prepare entry points; S tokens in all.
+int check_prepare(int dtype, int64_t S, int64_t D, const lcv_bsa_grid& rope, int64_t rope_table_len, float eps,
+                  const void* q_weight, const void* k_weight, const float* qbar, const float* kbar) {
+  if (rope.T <= 0 || rope.Hl <= 0 || rope.Wl <= 0 || rope.T * rope.Hl * rope.Wl != S)
+    return fail(LCV_BSA_ERR_SHAPE, "RoPE grid (%lld, %lld, %lld) must be positive with product S=%lld",
+                (long long)rope.T, (long long)rope.Hl, (long long)rope.Wl, (long long)S);
+  if (S > lcv::kPrepMaxTokens)
+    return fail(LCV_BSA_ERR_UNSUPPORTED, "prepare_qk supports at most %lld tokens (S=%lld)",
+                (long long)lcv::kPrepMaxTokens, (long long)S);
+  const int64_t need = lcv_bsa_rope_table_len(D, rope);
+  if (need == 0)
+    return fail(LCV_BSA_ERR_UNSUPPORTED, "RoPE table for this grid exceeds %d floats",
+                lcv::kMaxRopeTable);
+  if (rope_table_len != need)
+    return fail(LCV_BSA_ERR_INVALID_ARG, "rope_table_len=%lld, expected %lld",
+                (long long)rope_table_len, (long long)need);
+  if (!std::isfinite(eps) || eps < 0.0f) return fail(LCV_BSA_ERR_INVALID_ARG, "eps must be >= 0");
+  if ((uintptr_t)q_weight % 16 || (uintptr_t)k_weight % 16 || (uintptr_t)qbar % 16 ||
+      (uintptr_t)kbar % 16)
+    return fail(LCV_BSA_ERR_LAYOUT, "norm weights and block means must be 16-byte aligned");
+  return LCV_BSA_OK;
+}
+
+// Rows of one tensor of the prepare entry points: strides, 16-byte alignment.
+int check_rows(const char* name, const void* ptr, const lcv_bsa_strides& s, int64_t D) {
+  const int st = check_strides(name, s, D);
+  if (st) return st;
+  if (!vec_aligned(ptr, s, 8))
+    return fail(LCV_BSA_ERR_LAYOUT, "%s rows must start on 16-byte boundaries", name);
+  return LCV_BSA_OK;
+}
+
+lcv::Tensor4 tensor4(const void* ptr, const lcv_bsa_strides& s) { return {ptr, s.b, s.h, s.s}; }
+
+}  // namespace
+
+extern "C" {
+
 int lcv_bsa_prepare_qk(const void* q_in, const void* k_in, int dtype, int64_t B, int64_t H,
                        int64_t S, int64_t D, lcv_bsa_strides qis, lcv_bsa_strides kis,
                        const void* q_weight, const void* k_weight, float eps, lcv_bsa_grid rope,
@@ -748,39 +790,79 @@ int lcv_bsa_prepare_qk(const void* q_in, const void* k_in, int dtype, int64_t B,
   if (bs != 64)
     return fail(LCV_BSA_ERR_UNSUPPORTED, "prepare_qk requires 64-token blocks (got %lld)",
                 (long long)bs);
-  if (rope.T <= 0 || rope.Hl <= 0 || rope.Wl <= 0 || rope.T * rope.Hl * rope.Wl != S)
-    return fail(LCV_BSA_ERR_SHAPE, "RoPE grid (%lld, %lld, %lld) must be positive with product S=%lld",
-                (long long)rope.T, (long long)rope.Hl, (long long)rope.Wl, (long long)S);
-  if (S > lcv::kPrepMaxTokens)
-    return fail(LCV_BSA_ERR_UNSUPPORTED, "prepare_qk supports at most %lld tokens (S=%lld)",
-                (long long)lcv::kPrepMaxTokens, (long long)S);
-  const int64_t need = lcv_bsa_rope_table_len(D, rope);
-  if (need == 0)
-    return fail(LCV_BSA_ERR_UNSUPPORTED, "RoPE table for this grid exceeds %d floats",
-                lcv::kMaxRopeTable);
-  if (rope_table_len != need)
-    return fail(LCV_BSA_ERR_INVALID_ARG, "rope_table_len=%lld, expected %lld",
-                (long long)rope_table_len, (long long)need);
-  if (!std::isfinite(eps) || eps < 0.0f) return fail(LCV_BSA_ERR_INVALID_ARG, "eps must be >= 0");
-  if ((st = check_strides("q_in", qis, D)) || (st = check_strides("k_in", kis, D)) ||
-      (st = check_strides("q_out", qos, D)) || (st = check_strides("k_out", kos, D)))
+  if ((st = check_prepare(dtype, S, D, rope, rope_table_len, eps, q_weight, k_weight, qbar, kbar)) ||
+      (st = check_rows("q_in", q_in, qis, D)) || (st = check_rows("k_in", k_in, kis, D)) ||
+      (st = check_rows("q_out", q_out, qos, D)) || (st = check_rows("k_out", k_out, kos, D)))
     return st;
-  if (!vec_aligned(q_in, qis, 8) || !vec_aligned(k_in, kis, 8) || !vec_aligned(q_out, qos, 8) ||
-      !vec_aligned(k_out, kos, 8))
-    return fail(LCV_BSA_ERR_LAYOUT, "q/k rows must start on 16-byte boundaries");
-  if ((uintptr_t)q_weight % 16 || (uintptr_t)k_weight % 16 || (uintptr_t)qbar % 16 ||
-      (uintptr_t)kbar % 16)
-    return fail(LCV_BSA_ERR_LAYOUT, "norm weights and block means must be 16-byte aligned");
-  const lcv::Tensor4 in[2] = {{q_in, qis.b, qis.h, qis.s}, {k_in, kis.b, kis.h, kis.s}};
-  const lcv::Tensor4 out[2] = {{q_out, qos.b, qos.h, qos.s}, {k_out, kos.b, kos.h, kos.s}};
+  const lcv::Tensor4 in[2] = {tensor4(q_in, qis), tensor4(k_in, kis)};
+  const lcv::Tensor4 out[2] = {tensor4(q_out, qos), tensor4(k_out, kos)};
   const void* w[2] = {q_weight, k_weight};
   float* means[2] = {qbar, kbar};
   const int32_t grid[3] = {(int32_t)rope.T, (int32_t)rope.Hl, (int32_t)rope.Wl};
   const int32_t dims[2] = {(int32_t)(D - 4 * (D / 6)), (int32_t)(2 * (D / 6))};
   return launch_status(lcv::launch_prep(in, out, w, means, dtype, (int)B, (int)H, (int)D, (int)nb,
-                                        lcv::make_geom(g), grid, dims, rope_table, (int)need, eps,
+                                        lcv::make_geom(g), grid, dims, rope_table, (int)rope_table_len, eps,
                                         (hipStream_t)stream),
                        "lcv_bsa_prepare_qk");
+}
+
+int lcv_bsa_prepare_qkv(const void* q_in, const void* k_in, const void* v_in, int dtype, int64_t B,
+                        int64_t H, int64_t Sq, int64_t D, lcv_bsa_strides qis, lcv_bsa_strides kis,
+                        lcv_bsa_strides vis, const void* k_cache, const void* v_cache,
+                        int64_t S_cache, lcv_bsa_strides kcs, lcv_bsa_strides vcs,
+                        const void* q_weight, const void* k_weight, float eps, lcv_bsa_grid rope,
+                        const float* rope_table, int64_t rope_table_len, lcv_bsa_geom gq,
+                        lcv_bsa_geom gk, void* q_out, void* k_out, void* v_out, void* k_norm,
+                        lcv_bsa_strides qos, lcv_bsa_strides kos, lcv_bsa_strides vos,
+                        lcv_bsa_strides kns, float* qbar, float* kbar, void* stream) {
+  if (!q_in || !k_in || !q_out || !k_out || !qbar || !kbar || !rope_table)
+    return fail(LCV_BSA_ERR_INVALID_ARG, "null pointer");
+  if (S_cache < 0) return fail(LCV_BSA_ERR_INVALID_ARG, "S_cache must be >= 0");
+  if ((!v_in) != (!v_out) || (v_in && S_cache && !v_cache) || (S_cache && !k_cache))
+    return fail(LCV_BSA_ERR_INVALID_ARG, "v_in and v_out go together, and a cache of S_cache > 0 tokens with them");
+  if (!dtype_ok(dtype)) return fail(LCV_BSA_ERR_DTYPE, "unknown dtype %d", dtype);
+  if (!lcv::prep_supported(dtype, (int)D))
+    return fail(LCV_BSA_ERR_UNSUPPORTED, "prepare_qkv supports fp16/bf16 with D in {64, 128}");
+  int64_t nb = 0, bs = 0, nk = 0, bsk = 0;
+  int st = check_geom(B, H, Sq, D, gq, &nb, &bs);
+  if (st) return st;
+  if (S_cache > kI32Max / 4) return fail(LCV_BSA_ERR_UNSUPPORTED, "S_cache beyond 2^29");
+  const int64_t S = S_cache + Sq;
+  if ((st = check_geom(B, H, S, D, gk, &nk, &bsk))) return st;
+  if (bs != 64 || bsk != 64)
+    return fail(LCV_BSA_ERR_UNSUPPORTED, "prepare_qkv requires 64-token blocks (got %lld, %lld)",
+                (long long)bs, (long long)bsk);
+  if (3 * B * H * nk > kI32Max) return fail(LCV_BSA_ERR_UNSUPPORTED, "B*H*num_blocks too large");
+  if ((st = check_prepare(dtype, S, D, rope, rope_table_len, eps, q_weight, k_weight, qbar, kbar)) ||
+      (st = check_rows("q_in", q_in, qis, D)) || (st = check_rows("k_in", k_in, kis, D)) ||
+      (st = check_rows("q_out", q_out, qos, D)) || (st = check_rows("k_out", k_out, kos, D)) ||
+      (v_in && ((st = check_rows("v_in", v_in, vis, D)) || (st = check_rows("v_out", v_out, vos, D)))) ||
+      (S_cache && (st = check_rows("k_cache", k_cache, kcs, D))) ||
+      (S_cache && v_in && (st = check_rows("v_cache", v_cache, vcs, D))) ||
+      (k_norm && (st = check_rows("k_norm", k_norm, kns, D))))
+    return st;
+  lcv::PrepCached x{};
+  x.in[0] = tensor4(q_in, qis);
+  x.in[1] = tensor4(k_in, kis);
+  x.out[0] = tensor4(q_out, qos);
+  x.out[1] = tensor4(k_out, kos);
+  x.weight[0] = q_weight;
+  x.weight[1] = k_weight;
+  x.mean[0] = qbar;
+  x.mean[1] = kbar;
+  x.v_in = tensor4(v_in, vis);
+  x.v_out = tensor4(v_out, vos);
+  x.k_cache = tensor4(k_cache, kcs);
+  x.v_cache = tensor4(v_cache, vcs);
+  x.k_norm = tensor4(k_norm, kns);
+  x.cached = (int)S_cache;
+  const int32_t grid[3] = {(int32_t)rope.T, (int32_t)rope.Hl, (int32_t)rope.Wl};
+  const int32_t dims[2] = {(int32_t)(D - 4 * (D / 6)), (int32_t)(2 * (D / 6))};
+  return launch_status(lcv::launch_prep_cached(x, dtype, (int)B, (int)H, (int)D, (int)nb, (int)nk,
+                                               lcv::make_geom(gq), lcv::make_geom(gk), grid, dims,
+                                               rope_table, (int)rope_table_len, eps,
+                                               (hipStream_t)stream),
+                       "lcv_bsa_prepare_qkv");
 }
 
 }  // extern "C"

@@ -46,6 +46,20 @@ struct PrepArgs {
   FastDiv heads;          // H
 };
 
+// The cached form (prep_cached_kernel): k and v continue a cache of earlier
+// tokens, already normed and not yet rotated.
+struct CachedArgs {
+  PrepArgs p;             // in / out / weight / mean of q (0) and new k (1); g is q's geometry
+  Tensor4 cache[2];       // k, v of the cached tokens
+  Tensor4 v_in, v_out;    // new v, and cached + new v (null: v is not gathered)
+  Tensor4 k_norm;         // new k after its norm, before RoPE (null: not wanted)
+  int32_t cached;         // tokens in the cache
+  int32_t nk;             // blocks of k / v (cached + new)
+  int32_t head_items;     // items before the first q-block's
+  FastDiv head_per_block, bh;  // items per block among those, B * H
+  Geom gk;
+};
+
 // Quotient of n by d for n < 2^22 from an fp32 reciprocal: (n + 1/2) / d is
 // at least 1/(2d) away from an integer, more than the rounding error of
 // (n + 1/2) * fl(1/d) (under 2^-23 relative) can cover for n < 2^22.
@@ -69,6 +83,103 @@ __device__ __forceinline__ int lds_slot(const PrepArgs& a, int i) {
   }
   const int j = i - base;
   return j < n ? base + 2 * j : base + 2 * (j - n) + 1;
+}
+
+// What a lane needs to turn rows: per pair p (dims 8c + 2p, +1) its axis and its
+// column's offset in that axis' LDS row (in floats).
+template <int D>
+struct RopeLane {
+  int axis[4], col2[4];
+  int ht2, hh2, hw2;  // floats per LDS row of each axis
+  int reg_h, reg_w;
+  uint32_t plane;
+  __device__ RopeLane(const PrepArgs& a, int c) {
+    ht2 = a.dt, hh2 = a.dh, hw2 = D - a.dt - a.dh;
+    reg_h = a.rT * ht2, reg_w = reg_h + a.rH * hh2;
+#pragma unroll
+    for (int pp = 0; pp < 4; ++pp) {
+      const int d = 8 * c + 2 * pp;
+      axis[pp] = d < a.dt ? 0 : (d < a.dt + a.dh ? 1 : 2);
+      col2[pp] = axis[pp] == 0 ? d : (axis[pp] == 1 ? d - a.dt : d - a.dt - a.dh);
+    }
+    plane = (uint32_t)(a.rH * a.rW);
+  }
+};
+
+template <typename T>
+__device__ __forceinline__ u32x4 load_weight(const void* w, int c) {
+  if (w) return *reinterpret_cast<const u32x4*>(reinterpret_cast<const T*>(w) + 8 * c);
+  const uint32_t one = bits16(from_f32<T>(1.0f));
+  return u32x4{one | (one << 16), one | (one << 16), one | (one << 16), one | (one << 16)};
+}
+
+template <typename T>
+__device__ __forceinline__ void widen8(const u32x4& raw, float (&x)[8]) {
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    x[2 * m] = to_f32(__builtin_bit_cast(T, (uint16_t)(raw[m] & 0xffffu)));
+    x[2 * m + 1] = to_f32(__builtin_bit_cast(T, (uint16_t)(raw[m] >> 16)));
+  }
+}
+
+// RMSNorm of a row held 8 elements a lane over D / 8 lanes.
+template <typename T, int D>
+__device__ __forceinline__ void norm_row(const float (&x)[8], const u32x4& wr, float eps, float nz, float (&y)[8]) {
+  float ss = 0.0f;
+#pragma unroll
+  // x*x of a 16-bit value is exact in fp32, so the fused form rounds the
+  // sum exactly as square-then-add does.
+  for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(x[e], x[e], ss);
+  ss = group_sum<D / 8>(ss);
+  const float rs = rsqrtf(ss * (1.0f / D) + eps);
+  norm_scale<T>(x, rs, wr, nz, y);
+}
+
+// RoPE of y at grid position `tok`; the rounded row is packed and added to acc.
+template <typename T, int D>
+__device__ __forceinline__ u32x4 rope_row(const PrepArgs& a, const RopeLane<D>& L, const float* tab, uint32_t tok,
+                                          const float (&y)[8], float (&acc)[8]) {
+  const uint32_t pt = small_div(tok, a.rcp_plane);
+  const uint32_t prem = tok - __umul24(pt, L.plane);
+  const uint32_t ph = small_div(prem, a.rcp_w);
+  const uint32_t pw = prem - __umul24(ph, (uint32_t)a.rW);
+  const int at = (int)__umul24(pt, (uint32_t)L.ht2);
+  const int ah = L.reg_h + (int)__umul24(ph, (uint32_t)L.hh2);
+  const int aw = L.reg_w + (int)__umul24(pw, (uint32_t)L.hw2);
+  const float nz = a.neg_zero, one = a.one;
+  uint32_t packed[4];
+#pragma unroll
+  for (int pp = 0; pp < 4; ++pp) {
+    const int slot = (L.axis[pp] == 0 ? at : (L.axis[pp] == 1 ? ah : aw)) + L.col2[pp];
+    const float2 f = *reinterpret_cast<const float2*>(tab + slot);
+    const float cs = f.x, sn = f.y;
+    const float u = y[2 * pp], v = y[2 * pp + 1];
+    // x*cos + rotate_half(x)*sin, rounded per product and sum.
+    const T o0 = round_from_f32<T>(mul1(u, cs, nz) - mul1(v, sn, nz));
+    const T o1 = round_from_f32<T>(mul1(v, cs, nz) + mul1(u, sn, nz));
+    acc[2 * pp] = __builtin_fmaf(to_f32(o0), one, acc[2 * pp]);
+    acc[2 * pp + 1] = __builtin_fmaf(to_f32(o1), one, acc[2 * pp + 1]);
+    packed[pp] = bits16(o0) | (bits16(o1) << 16);
+  }
+  return u32x4{packed[0], packed[1], packed[2], packed[3]};
+}
+
+// Block mean: combine the row groups (lanes c, c + LPR, ...) in a fixed
+// butterfly order; the lanes of group 0 store the D means.
+template <int D>
+__device__ __forceinline__ void store_mean(float (&acc)[8], float* mean, int lane) {
+  constexpr int LPR = D / 8;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+#pragma unroll
+    for (int m = LPR; m < 64; m <<= 1) acc[e] += __shfl_xor(acc[e], m);
+  }
+  if (lane < LPR) {
+    float* mp = mean + 8 * lane;
+    constexpr float inv = 1.0f / 64.0f;
+    *reinterpret_cast<float4*>(mp) = float4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
+    *reinterpret_cast<float4*>(mp + 4) = float4{acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv};
+  }
 }
 
 template <typename T, int D>
@@ -97,19 +208,7 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
   const int wave = uniform_i32(threadIdx.x / 64);
   const int lane = threadIdx.x % 64;
   const int c = lane % LPR;  // this lane's 8 dims: 8c .. 8c+7
-  // Per pair p (dims 8c + 2p, +1): its axis and its column's offset in that
-  // axis' LDS row (in floats).
-  const int ht2 = a.dt, hh2 = a.dh, hw2 = D - a.dt - a.dh;  // floats per LDS row
-  const int reg_h = a.rT * ht2, reg_w = reg_h + a.rH * hh2;
-  int axis[4], col2[4];
-#pragma unroll
-  for (int pp = 0; pp < 4; ++pp) {
-    const int d = 8 * c + 2 * pp;
-    axis[pp] = d < a.dt ? 0 : (d < a.dt + a.dh ? 1 : 2);
-    col2[pp] = axis[pp] == 0 ? d : (axis[pp] == 1 ? d - a.dt : d - a.dt - a.dh);
-  }
-  const uint32_t plane = (uint32_t)(a.rH * a.rW);
-  const float nz = a.neg_zero, one = a.one;
+  const RopeLane<D> L(a, c);
   const int stride = gridDim.x * kPrepWaves;
 
   for (int item = blockIdx.x * kPrepWaves + wave; item < a.total_items; item += stride) {
@@ -129,13 +228,7 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
                    (int64_t)tok0 * xi.ss + 8 * c;
     T* dst = reinterpret_cast<T*>(const_cast<void*>(xo.ptr)) + (int64_t)b * xo.sb + (int64_t)h * xo.sh +
              (int64_t)tok0 * xo.ss + 8 * c;
-    u32x4 wr;
-    if (a.weight[tensor]) {
-      wr = *reinterpret_cast<const u32x4*>(reinterpret_cast<const T*>(a.weight[tensor]) + 8 * c);
-    } else {
-      const uint32_t one = bits16(from_f32<T>(1.0f));
-      wr = u32x4{one | (one << 16), one | (one << 16), one | (one << 16), one | (one << 16)};
-    }
+    const u32x4 wr = load_weight<T>(a.weight[tensor], c);
 
     float acc[8];
 #pragma unroll
@@ -145,88 +238,144 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
       const int row = st * RPS + lane / LPR;
       // q / k are streamed once: non-temporal loads and stores.
       const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + row_in[tensor][row]));
-      float x[8];
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        x[2 * m] = to_f32(__builtin_bit_cast(T, (uint16_t)(raw[m] & 0xffffu)));
-        x[2 * m + 1] = to_f32(__builtin_bit_cast(T, (uint16_t)(raw[m] >> 16)));
-      }
-      // RMSNorm: the row's sum of squares over its LPR lanes.
-      float ss = 0.0f;
-#pragma unroll
-      // x*x of a 16-bit value is exact in fp32, so the fused form rounds the
-      // sum exactly as square-then-add does.
-      for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(x[e], x[e], ss);
-      ss = group_sum<LPR>(ss);
-      const float rs = rsqrtf(ss * (1.0f / D) + a.eps);
-      float y[8];
-      norm_scale<T>(x, rs, wr, nz, y);
-      // RoPE at the token's grid position: the LDS row of each axis.
-      const uint32_t tok = (uint32_t)(tok0 + row_tok[row]);
-      const uint32_t pt = small_div(tok, a.rcp_plane);
-      const uint32_t prem = tok - __umul24(pt, plane);
-      const uint32_t ph = small_div(prem, a.rcp_w);
-      const uint32_t pw = prem - __umul24(ph, (uint32_t)a.rW);
-      const int at = (int)__umul24(pt, (uint32_t)ht2);
-      const int ah = reg_h + (int)__umul24(ph, (uint32_t)hh2);
-      const int aw = reg_w + (int)__umul24(pw, (uint32_t)hw2);
-      uint32_t packed[4];
-#pragma unroll
-      for (int pp = 0; pp < 4; ++pp) {
-        const int slot = (axis[pp] == 0 ? at : (axis[pp] == 1 ? ah : aw)) + col2[pp];
-        const float2 f = *reinterpret_cast<const float2*>(tab + slot);
-        const float cs = f.x, sn = f.y;
-        const float u = y[2 * pp], v = y[2 * pp + 1];
-        // x*cos + rotate_half(x)*sin, rounded per product and sum.
-        const T o0 = round_from_f32<T>(mul1(u, cs, nz) - mul1(v, sn, nz));
-        const T o1 = round_from_f32<T>(mul1(v, cs, nz) + mul1(u, sn, nz));
-        acc[2 * pp] = __builtin_fmaf(to_f32(o0), one, acc[2 * pp]);
-        acc[2 * pp + 1] = __builtin_fmaf(to_f32(o1), one, acc[2 * pp + 1]);
-        packed[pp] = bits16(o0) | (bits16(o1) << 16);
-      }
-      __builtin_nontemporal_store(u32x4{packed[0], packed[1], packed[2], packed[3]},
-                                  reinterpret_cast<u32x4*>(dst + row_out[tensor][row]));
+      float x[8], y[8];
+      widen8<T>(raw, x);
+      norm_row<T, D>(x, wr, a.eps, a.neg_zero, y);
+      const u32x4 packed = rope_row<T, D>(a, L, tab, (uint32_t)(tok0 + row_tok[row]), y, acc);
+      __builtin_nontemporal_store(packed, reinterpret_cast<u32x4*>(dst + row_out[tensor][row]));
     }
-    // Block mean: combine the RPS row groups (lanes c, c+LPR, ...) in a fixed
-    // butterfly order; the lanes of group 0 store the D means.
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-#pragma unroll
-      for (int m = LPR; m < 64; m <<= 1) acc[e] += __shfl_xor(acc[e], m);
-    }
-    if (lane < LPR) {
-      float* mp = a.mean[tensor] + ((int64_t)bh * a.nb + n) * D + 8 * c;
-      constexpr float inv = 1.0f / 64.0f;
-      *reinterpret_cast<float4*>(mp) = float4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
-      *reinterpret_cast<float4*>(mp + 4) = float4{acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv};
-    }
+    store_mean<D>(acc, a.mean[tensor] + ((int64_t)bh * a.nb + n) * D, lane);
   }
+}
+
+// prep_kernel with q and k of different lengths: k (and v) rows below `cached`
+// come from the cache, k's un-normed; RoPE positions run over cached + new
+// tokens, so new row r of q and k sits at cached + r.  q is read once, cached and
+// new k once, and nothing is padded, concatenated or rotated in between.  Items
+// run k-block (v-block) by k-block; the last nb of the nk k-blocks go with the
+// q-blocks, so that the rows of a token that q, k and v share are read together.
+// HBM bound, as prep_kernel.  Measured at 32 heads of 128, bf16, 3,600 tokens a
+// frame: 8 frames after 4 cached ones 1.89 GB in 0.40 ms, 4.7 TB/s (the torch
+// norms, concatenations and RoPE it replaces: 7.3 ms); filling a cache of 4
+// frames 0.59 GB in 0.15 ms (2.3 ms).
+template <typename T, int D>
+__global__ __launch_bounds__(256) void prep_cached_kernel(CachedArgs ca) {
+  constexpr int LPR = D / 8;
+  constexpr int RPS = 64 / LPR;
+  extern __shared__ float tab[];
+  __shared__ int32_t row_tok[2][64];  // token offset of each block row: q's geometry, k's
+  const PrepArgs& a = ca.p;
+  for (int i = threadIdx.x; i < a.table_len; i += 256) tab[lds_slot(a, i)] = a.table[i];
+  if (threadIdx.x < 64) {
+    row_tok[0][threadIdx.x] = voxel_row_offset(a.g, threadIdx.x);
+    row_tok[1][threadIdx.x] = voxel_row_offset(ca.gk, threadIdx.x);
+  }
+  __syncthreads();
+  const int wave = uniform_i32(threadIdx.x / 64);
+  const int lane = threadIdx.x % 64;
+  const int c = lane % LPR;
+  const RopeLane<D> L(a, c);
+  const int stride = gridDim.x * kPrepWaves;
+
+  for (int item = blockIdx.x * kPrepWaves + wave; item < a.total_items; item += stride) {
+    int tensor, n;   // 0 q, 1 k, 2 v; its block
+    uint32_t r;
+    if (item < ca.head_items) {
+      n = (int)fast_div((uint32_t)item, ca.head_per_block);
+      r = (uint32_t)item - (uint32_t)n * ca.head_per_block.d;
+      tensor = 1 + (int)fast_div(r, ca.bh);
+      r -= (uint32_t)(tensor - 1) * ca.bh.d;
+    } else {
+      const uint32_t it = (uint32_t)(item - ca.head_items);
+      n = (int)fast_div(it, a.per_block);
+      r = it - (uint32_t)n * a.per_block.d;
+      tensor = (int)fast_div(r, ca.bh);
+      r -= (uint32_t)tensor * ca.bh.d;
+      if (tensor) n += ca.nk - a.nb;
+    }
+    const int bh = (int)r;
+    const int b = (int)fast_div(r, a.heads);
+    const int h = bh - b * (int)a.heads.d;
+    const int32_t tok0 = block_base_token(tensor ? ca.gk : a.g, n);
+    const Tensor4 xi = tensor == 2 ? ca.v_in : a.in[tensor];
+    const Tensor4 xo = tensor == 2 ? ca.v_out : a.out[tensor];
+    const Tensor4 xc = ca.cache[tensor == 2 ? 1 : 0];
+    const int first_new = tensor ? ca.cached : 0;  // rows below come from the cache
+    const T* src = reinterpret_cast<const T*>(xi.ptr) + (int64_t)b * xi.sb + (int64_t)h * xi.sh + 8 * c;
+    const T* old = reinterpret_cast<const T*>(xc.ptr) + (int64_t)b * xc.sb + (int64_t)h * xc.sh + 8 * c;
+    T* dst = reinterpret_cast<T*>(const_cast<void*>(xo.ptr)) + (int64_t)b * xo.sb + (int64_t)h * xo.sh + 8 * c;
+    const int32_t* rows = row_tok[tensor ? 1 : 0];
+    if (tensor == 2) {
+#pragma unroll 4
+      for (int st = 0; st < 64 / RPS; ++st) {
+        const int32_t t = tok0 + rows[st * RPS + lane / LPR];
+        const T* from = t < first_new ? old + (int64_t)t * xc.ss : src + (int64_t)(t - first_new) * xi.ss;
+        __builtin_nontemporal_store(__builtin_nontemporal_load(reinterpret_cast<const u32x4*>(from)),
+                                    reinterpret_cast<u32x4*>(dst + (int64_t)t * xo.ss));
+      }
+      continue;
+    }
+    T* kn = tensor && ca.k_norm.ptr ? reinterpret_cast<T*>(const_cast<void*>(ca.k_norm.ptr)) +
+                                          (int64_t)b * ca.k_norm.sb + (int64_t)h * ca.k_norm.sh + 8 * c
+                                    : nullptr;
+    const u32x4 wr = load_weight<T>(a.weight[tensor], c);
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
+#pragma unroll 2
+    for (int st = 0; st < 64 / RPS; ++st) {
+      const int32_t t = tok0 + rows[st * RPS + lane / LPR];
+      const bool is_new = t >= first_new;
+      const T* from = is_new ? src + (int64_t)(t - first_new) * xi.ss : old + (int64_t)t * xc.ss;
+      const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(from));
+      float x[8], y[8];
+      widen8<T>(raw, x);
+      norm_row<T, D>(x, wr, a.eps, a.neg_zero, y);
+      if (kn && is_new) {
+        uint32_t w[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m)  // exact: y holds T values
+          w[m] = bits16(from_f32<T>(y[2 * m])) | (bits16(from_f32<T>(y[2 * m + 1])) << 16);
+        *reinterpret_cast<u32x4*>(kn + (int64_t)(t - first_new) * ca.k_norm.ss) = u32x4{w[0], w[1], w[2], w[3]};
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = is_new ? y[e] : x[e];
+      const uint32_t pos = (uint32_t)(tensor ? t : t + ca.cached);
+      const u32x4 packed = rope_row<T, D>(a, L, tab, pos, y, acc);
+      __builtin_nontemporal_store(packed, reinterpret_cast<u32x4*>(dst + (int64_t)t * xo.ss));
+    }
+    store_mean<D>(acc, a.mean[tensor] + ((int64_t)bh * (tensor ? ca.nk : a.nb) + n) * D, lane);
+  }
+}
+
+// As many workgroups as are resident at once (each stages the table once).
+template <typename Args>
+hipError_t launch_resident(void (*kernel)(Args), const Args& args, int table_len, int items, hipStream_t stream) {
+  const size_t shmem = (size_t)table_len * sizeof(float);
+  int dev = 0, cus = 0, per_cu = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 256, shmem);
+  if (e != hipSuccess) return e;
+  const int want = (items + kPrepWaves - 1) / kPrepWaves;
+  const int grid = std::max(1, std::min(want, cus * std::max(per_cu, 1)));
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), shmem, stream, args);
+  return hipGetLastError();
 }
 
 template <typename T, int D>
 hipError_t launch_prep_t(const PrepArgs& a, hipStream_t stream) {
-  const size_t shmem = (size_t)a.table_len * sizeof(float);
-  int dev = 0, cus = 0, per_cu = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e == hipSuccess)
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, prep_kernel<T, D>, 256, shmem);
-  if (e != hipSuccess) return e;
-  // As many workgroups as are resident at once (each stages the table once).
-  const int want = (a.total_items + kPrepWaves - 1) / kPrepWaves;
-  const int grid = std::max(1, std::min(want, cus * std::max(per_cu, 1)));
-  hipLaunchKernelGGL((prep_kernel<T, D>), dim3(grid), dim3(256), shmem, stream, a);
-  return hipGetLastError();
+  return launch_resident(&prep_kernel<T, D>, a, a.table_len, a.total_items, stream);
 }
 
-}  // namespace
+template <typename T, int D>
+hipError_t launch_cached_t(const CachedArgs& a, hipStream_t stream) {
+  return launch_resident(&prep_cached_kernel<T, D>, a, a.p.table_len, a.p.total_items, stream);
+}
 
-bool prep_supported(int dtype, int D) { return dtype != 2 && (D == 64 || D == 128); }
-
-hipError_t launch_prep(const Tensor4* in, const Tensor4* out, const void* const* weight,
-                       float* const* mean, int dtype, int B, int H, int D, int nb, const Geom& g,
-                       const int32_t* rope_grid, const int32_t* rope_dims, const float* table,
-                       int table_len, float eps, hipStream_t stream) {
+PrepArgs prep_args(const Tensor4* in, const Tensor4* out, const void* const* weight, float* const* mean, int H, int D,
+                   int nb, const Geom& g, const int32_t* rope_grid, const int32_t* rope_dims, const float* table,
+                   int table_len, float eps) {
   PrepArgs a{};
   for (int t = 0; t < 2; ++t) {
     a.in[t] = in[t];
@@ -244,17 +393,52 @@ hipError_t launch_prep(const Tensor4* in, const Tensor4* out, const void* const*
   a.dt = rope_dims[0];
   a.dh = rope_dims[1];
   a.table_len = table_len;
-  a.total_items = 2 * B * H * nb;
   a.eps = eps;
   a.g = g;
-  a.per_block = make_fastdiv((uint32_t)(2 * B * H));
   a.heads = make_fastdiv((uint32_t)H);
   a.rcp_plane = (float)(1.0 / ((double)a.rH * a.rW));
   a.rcp_w = (float)(1.0 / (double)a.rW);
   a.neg_zero = -0.0f;
   a.one = 1.0f;
+  return a;
+}
+
+}  // namespace
+
+bool prep_supported(int dtype, int D) { return dtype != 2 && (D == 64 || D == 128); }
+
+hipError_t launch_prep(const Tensor4* in, const Tensor4* out, const void* const* weight,
+                       float* const* mean, int dtype, int B, int H, int D, int nb, const Geom& g,
+                       const int32_t* rope_grid, const int32_t* rope_dims, const float* table,
+                       int table_len, float eps, hipStream_t stream) {
+  PrepArgs a = prep_args(in, out, weight, mean, H, D, nb, g, rope_grid, rope_dims, table, table_len, eps);
+  a.total_items = 2 * B * H * nb;
+  a.per_block = make_fastdiv((uint32_t)(2 * B * H));
   if (dtype == 0) return D == 128 ? launch_prep_t<f16, 128>(a, stream) : launch_prep_t<f16, 64>(a, stream);
   return D == 128 ? launch_prep_t<bf16, 128>(a, stream) : launch_prep_t<bf16, 64>(a, stream);
+}
+
+hipError_t launch_prep_cached(const PrepCached& x, int dtype, int B, int H, int D, int nb, int nk, const Geom& g,
+                              const Geom& gk, const int32_t* rope_grid, const int32_t* rope_dims, const float* table,
+                              int table_len, float eps, hipStream_t stream) {
+  CachedArgs c{};
+  c.p = prep_args(x.in, x.out, x.weight, x.mean, H, D, nb, g, rope_grid, rope_dims, table, table_len, eps);
+  c.cache[0] = x.k_cache;
+  c.cache[1] = x.v_cache;
+  c.v_in = x.v_in;
+  c.v_out = x.v_out;
+  c.k_norm = x.k_norm;
+  c.cached = x.cached;
+  c.nk = nk;
+  c.gk = gk;
+  const int kv = x.v_out.ptr ? 2 : 1;  // tensors over the k-blocks
+  c.head_items = (nk - nb) * kv * B * H;
+  c.head_per_block = make_fastdiv((uint32_t)(kv * B * H));
+  c.bh = make_fastdiv((uint32_t)(B * H));
+  c.p.per_block = make_fastdiv((uint32_t)((kv + 1) * B * H));
+  c.p.total_items = c.head_items + (kv + 1) * B * H * nb;
+  if (dtype == 0) return D == 128 ? launch_cached_t<f16, 128>(c, stream) : launch_cached_t<f16, 64>(c, stream);
+  return D == 128 ? launch_cached_t<bf16, 128>(c, stream) : launch_cached_t<bf16, 64>(c, stream);
 }
 
 }  // namespace lcv

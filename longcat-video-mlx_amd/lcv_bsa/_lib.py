@@ -91,6 +91,11 @@ _SIGNATURES = {
                                    Strides, Strides, c_void_p, c_void_p, c_float, Grid, c_void_p,
                                    c_int64, Geom, c_void_p, c_void_p, Strides, Strides, c_void_p,
                                    c_void_p, c_void_p]),
+    "lcv_bsa_prepare_qkv": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64,
+                                    Strides, Strides, Strides, c_void_p, c_void_p, c_int64, Strides, Strides,
+                                    c_void_p, c_void_p, c_float, Grid, c_void_p, c_int64, Geom, Geom,
+                                    c_void_p, c_void_p, c_void_p, c_void_p, Strides, Strides, Strides, Strides,
+                                    c_void_p, c_void_p, c_void_p]),
 }
 
 EXPORTED = tuple(_SIGNATURES)

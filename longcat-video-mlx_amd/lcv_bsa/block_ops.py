@@ -17,7 +17,25 @@ import torch
 from . import _lib
 from .block_sparse_attention import _dtype_code, _require_device, _stream, _strides
 
-__all__ = ["residual_norm", "swiglu", "head_rms_norm"]
+__all__ = ["residual_norm", "swiglu", "head_rms_norm", "plain_tensors"]
+
+
+def plain_tensors(*ts: Optional[torch.Tensor]) -> bool:
+    """Whether a chain of torch operations over these GPU tensors (None skipped)
+    may run as one kernel that autograd and torch's tracers do not see: 16-bit
+    tensors of one dtype on one device, no gradient wanted from them (reverse or
+    forward mode), no transform, trace or tensor subclass looking on."""
+    ts = [t for t in ts if t is not None]
+    t0 = ts[0]
+    if not t0.is_cuda or t0.dtype not in (torch.float16, torch.bfloat16):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+        return False
+    if (torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0):
+        return False
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == t0.dtype and t.device == t0.device
+               for t in ts)
 
 
 def _ptr(t: Optional[torch.Tensor]):

@@ -24,10 +24,10 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .attention import BSAAttention, dense_attention, validate_backend
-from .block_ops import head_rms_norm, residual_norm, swiglu
+from .block_ops import head_rms_norm, plain_tensors, residual_norm, swiglu
 from .block_sparse_attention import bsa_attention
 from .block_sparse_attention_hip import bsa_attention_hip
-from .prepare import prepare_qk
+from .prepare import prepare_qk, prepare_qkv
 from .rope_3d import rope_3d
 from .shape_policy import bsa_geometry
 
@@ -123,11 +123,12 @@ class Attention(nn.Module, BSAAttention):
     reference always runs dense attention; ``bsa_cond_noise = True`` runs BSA
     there too (k-blocks over the longer key grid).
 
-    With BSA on and no KV cache to return, q and k go through one
-    ``prepare_qk`` over the strided views of the QKV output (RMSNorm + RoPE +
-    block means), and the attention writes straight into the ``[B, N, H, D]``
-    layout of the output projection.  A ``ValueError`` anywhere on that path
-    falls back to the reference's unfused sequence."""
+    With BSA on, q and k go through one ``prepare_qk`` over the strided views
+    of the QKV output (RMSNorm + RoPE + block means), and the attention writes
+    straight into the ``[B, N, H, D]`` layout of the output projection; around
+    a KV cache (returned, or continued) ``prepare_qkv`` does the same where no
+    gradient is wanted through the cache.  A ``ValueError`` anywhere on that
+    path falls back to the reference's unfused sequence."""
 
     def __init__(self, dim: int, num_heads: int, **kw):
         nn.Module.__init__(self)
@@ -188,19 +189,25 @@ class Attention(nn.Module, BSAAttention):
         qkv = self.qkv(x).view(B, N, 3, H, D)
         q, k, v = (qkv[:, :, i].transpose(1, 2) for i in range(3))
         o = torch.empty((B, N, H, D), dtype=x.dtype, device=x.device)
-        if self.enable_bsa and shape is not None and not return_kv:
+        if (self.enable_bsa and shape is not None
+                and (not return_kv or self._cache_fusible(qkv))):
             validate_backend(self.bsa_backend)
             geom = bsa_geometry(shape, self.bsa_chunk_thw, self.bsa_shape_policy)
             if geom is not None:
+                weights = dict(q_weight=self.q_norm.weight, k_weight=self.k_norm.weight, eps=self.q_norm.eps)
                 try:
-                    qp, kp, qb, kb = prepare_qk(q, k, shape, q_weight=self.q_norm.weight,
-                                                k_weight=self.k_norm.weight, eps=self.q_norm.eps,
-                                                shape=geom[0], chunk_thw=geom[1])
+                    if return_kv:
+                        kn = torch.empty((B, N, H, D), dtype=k.dtype, device=k.device).transpose(1, 2)
+                        qp, kp, _, qb, kb = prepare_qkv(q, k, None, shape, geom[0], geom[0], geom[1], k_norm=kn,
+                                                        **weights)
+                    else:
+                        qp, kp, qb, kb = prepare_qk(q, k, shape, shape=geom[0], chunk_thw=geom[1], **weights)
                     if ncl > 0:
                         self._split(qp, kp, v, shape, ncl, o)
                     else:
                         self._attend("all", qp, kp, v, shape, means=(qb, kb), out=o.transpose(1, 2))
-                    return self.proj(o.view(B, N, C))
+                    out = self.proj(o.view(B, N, C))
+                    return (out, (kn, v)) if return_kv else out
                 except ValueError:
                     self.last_indices, self.last_paths = {}, {}
         # The reference's sequence: norms, (cache,) RoPE, then BSA-or-dense.
@@ -214,6 +221,39 @@ class Attention(nn.Module, BSAAttention):
         out = self.proj(o.view(B, N, C))
         return (out, cache) if return_kv else out
 
+    def _cache_fusible(self, *tensors) -> bool:
+        """The norms around a KV cache as one kernel: nothing differentiates or
+        traces through them, and both round and weigh alike."""
+        return (self.q_norm.eps == self.k_norm.eps
+                and plain_tensors(*tensors, self.q_norm.weight, self.k_norm.weight))
+
+    def _continue_fused(self, q, k, v, x, shape, ncl, kv_cache):
+        """The continuation with BSA over cached + new keys, from one
+        ``prepare_qkv``; None where it does not apply."""
+        k_cache, v_cache = kv_cache
+        T, Hl, Wl = (int(s) for s in shape)
+        B, H, N, D = q.shape
+        if not (self.enable_bsa and self.bsa_cond_noise and ncl > 0 and N == T * Hl * Wl
+                and tuple(k_cache.shape) == tuple(v_cache.shape) == (k_cache.shape[0], H, ncl * Hl * Wl, D)
+                and k_cache.shape[0] in (1, B)
+                and self._cache_fusible(q, k_cache, v_cache)):
+            return None
+        validate_backend(self.bsa_backend)
+        grid = (T + ncl, Hl, Wl)
+        gq, gk = (bsa_geometry(g, self.bsa_chunk_thw, self.bsa_shape_policy) for g in ((T, Hl, Wl), grid))
+        if gq is None or gk is None or gq[1] != gk[1]:
+            return None
+        try:
+            q, k, v, qb, kb = prepare_qkv(q, k, v, grid, gq[0], gk[0], gq[1], cache=(k_cache, v_cache),
+                                          q_weight=self.q_norm.weight, k_weight=self.k_norm.weight,
+                                          eps=self.q_norm.eps)
+        except ValueError:
+            return None
+        self.last_indices, self.last_paths = {}, {}
+        o = torch.empty((B, N, H, D), dtype=x.dtype, device=x.device)
+        self._attend("noise", q, k, v, (T, Hl, Wl), kv_shape=grid, means=(qb, kb), out=o.transpose(1, 2))
+        return self.proj(o.view(B, N, H * D))
+
     def forward_with_kv_cache(self, x: torch.Tensor, shape: Sequence[int], num_cond_latents: Optional[int],
                               kv_cache: tuple) -> torch.Tensor:
         """Chunked continuation (attention.py:235-275): fresh k / v appended to
@@ -224,6 +264,9 @@ class Attention(nn.Module, BSAAttention):
         H, D = self.num_heads, self.head_dim
         qkv = self.qkv(x).view(B, N, 3, H, D)
         q, k, v = (qkv[:, :, i].transpose(1, 2) for i in range(3))
+        fused = self._continue_fused(q, k, v, x, shape, int(num_cond_latents or 0), kv_cache)
+        if fused is not None:
+            return fused
         q, k = self.q_norm(q), self.k_norm(k)
         T, Hl, Wl = (int(s) for s in shape)
         k_cache, v_cache = kv_cache

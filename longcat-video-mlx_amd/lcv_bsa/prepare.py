@@ -33,7 +33,7 @@ from .block_sparse_attention import (
 )
 from .rope_3d import BASE, rope_dims
 
-__all__ = ["rope_table", "prepare_qk", "RMS_EPS"]
+__all__ = ["rope_table", "prepare_qk", "prepare_qkv", "RMS_EPS"]
 
 RMS_EPS = 1e-6  # q_norm / k_norm, attention.py:53-54
 
@@ -46,6 +46,7 @@ def _axis_table(dim: int, n: int, device) -> tuple[torch.Tensor, torch.Tensor]:
 
 
 _TABLES: dict = {}
+_MAX_TABLES = 256  # of at most 48 KB; none is dropped, so a kernel in flight keeps the one it reads
 
 
 def rope_table(head_dim: int, grid: Sequence[int], device=None) -> torch.Tensor:
@@ -54,14 +55,24 @@ def rope_table(head_dim: int, grid: Sequence[int], device=None) -> torch.Tensor:
 
     Built once per (head_dim, grid, device) and kept: the kernel only reads
     it, and building it takes about thirty small launches (~0.15 ms at
-    720p), which would otherwise recur in every attention layer."""
+    720p), which would otherwise recur in every attention layer.  A table is
+    complete before it is kept, so that any stream may read it; one built under
+    stream capture belongs to that graph and is not kept."""
     dev = torch.device(device) if device is not None else torch.device("cpu")
     if dev.type == "cuda" and dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
     key = (int(head_dim), tuple(int(x) for x in grid), dev)
     table = _TABLES.get(key)
     if table is None:
-        table = _TABLES[key] = _build_table(head_dim, grid, dev)
+        table = _build_table(head_dim, grid, dev)
+        if dev.type == "cuda":
+            stream = torch.cuda.current_stream(dev)
+            with torch.cuda.device(dev):
+                if torch.cuda.is_current_stream_capturing():
+                    return table
+            stream.synchronize()
+        if len(_TABLES) < _MAX_TABLES:
+            _TABLES[key] = table
     return table
 
 
@@ -72,6 +83,28 @@ def _build_table(head_dim: int, grid: Sequence[int], device) -> torch.Tensor:
     for dim, n in ((dt, T), (dh, Hl), (dw, Wl)):
         parts.extend(_axis_table(dim, n, device))
     return torch.cat(parts).contiguous()
+
+
+def _norm_weights(ws, q: torch.Tensor):
+    D = q.shape[-1]
+    for w in ws:
+        if w is not None and w.shape != (D,):
+            raise ValueError(f"norm weight must be [{D}], got {tuple(w.shape)}")
+    return [None if w is None else w.to(device=q.device, dtype=q.dtype).contiguous() for w in ws]
+
+
+def _device_table(lib, D: int, g, grid: Sequence[int], device) -> torch.Tensor:
+    n_tab = lib.lcv_bsa_rope_table_len(D, g)
+    if n_tab == 0:
+        raise ValueError(f"prepare_qk supports D in {{64, 128}} and RoPE grids up to the table limit "
+                         f"(D={D}, grid={tuple(grid)})")
+    table = rope_table(D, grid, device)
+    assert table.numel() == n_tab
+    return table
+
+
+def _ptr(t: Optional[torch.Tensor]):
+    return None if t is None else t.data_ptr()
 
 
 def prepare_qk(
@@ -102,22 +135,10 @@ def prepare_qk(
     _check_shape(S, shape, chunk_thw)
     code = _dtype_code(q)
     q, k = _aligned_rows(q), _aligned_rows(k)
-    weights = []
-    for w in (q_weight, k_weight):
-        if w is None:
-            weights.append(None)
-            continue
-        if w.shape != (D,):
-            raise ValueError(f"norm weight must be [{D}], got {tuple(w.shape)}")
-        weights.append(w.to(device=q.device, dtype=q.dtype).contiguous())
+    weights = _norm_weights((q_weight, k_weight), q)
     lib = _lib.load()
     g = _lib.Grid(*(int(x) for x in grid))
-    n_tab = lib.lcv_bsa_rope_table_len(D, g)
-    if n_tab == 0:
-        raise ValueError(f"prepare_qk supports D in {{64, 128}} and RoPE grids up to the table limit "
-                         f"(D={D}, grid={tuple(grid)})")
-    table = rope_table(D, grid, q.device)
-    assert table.numel() == n_tab
+    table = _device_table(lib, D, g, grid, q.device)
     nb = num_blocks(shape, chunk_thw)
     q_out = torch.empty((B, H, S, D), dtype=q.dtype, device=q.device)
     k_out = torch.empty_like(q_out)
@@ -125,11 +146,85 @@ def prepare_qk(
     k_blocks = torch.empty_like(q_blocks)
     st = lib.lcv_bsa_prepare_qk(
         q.data_ptr(), k.data_ptr(), code, B, H, S, D, _strides(q), _strides(k),
-        weights[0].data_ptr() if weights[0] is not None else None,
-        weights[1].data_ptr() if weights[1] is not None else None,
-        float(eps), g, table.data_ptr(), n_tab, _geom(shape, chunk_thw),
+        _ptr(weights[0]), _ptr(weights[1]), float(eps), g, table.data_ptr(), table.numel(), _geom(shape, chunk_thw),
         q_out.data_ptr(), k_out.data_ptr(), _strides(q_out), _strides(k_out),
         q_blocks.data_ptr(), k_blocks.data_ptr(), _stream(q),
     )
     _lib.check(st, "prepare_qk")
     return q_out, k_out, q_blocks, k_blocks
+
+
+def prepare_qkv(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: Optional[torch.Tensor],
+    grid: Sequence[int],
+    shape: Sequence[int],
+    kv_shape: Sequence[int],
+    chunk_thw: Sequence[int],
+    *,
+    cache: Optional[tuple[torch.Tensor, torch.Tensor]] = None,
+    k_norm: Optional[torch.Tensor] = None,
+    q_weight: Optional[torch.Tensor] = None,
+    k_weight: Optional[torch.Tensor] = None,
+    eps: float = RMS_EPS,
+):
+    """``prepare_qk`` around a KV cache, in one pass (``lcv_bsa_prepare_qkv``).
+
+    ``cache=(k, v)`` holds the normed, un-rotated k and the v of earlier tokens
+    (``[B or 1, H, S_c, D]``) that the new ``q, k, v`` ``[B, H, S, D]`` follow;
+    ``grid`` is the latent grid of all ``S_c + S`` tokens, ``shape`` / ``kv_shape``
+    the BSA geometries of q and of cached + new k.  Without a cache ``v`` may be
+    None.  ``k_norm``, if given, receives the new k after its norm and before
+    RoPE: what a cache holds.
+
+    Returns ``(q_out, k_out, v_out, q_blocks, k_blocks)`` with k_out and v_out
+    over ``S_c + S`` tokens (v_out None when v is).
+    """
+    _require_device(q, k, *([] if v is None else [v]), *(cache or ()), *([] if k_norm is None else [k_norm]))
+    q, k = _bhsd(q, "q"), _bhsd(k, "k")
+    v = None if v is None else _bhsd(v, "v")
+    B, H, S, D = q.shape
+    cached = cache[0].shape[2] if cache is not None else 0
+    full = (B, H, cached + S, D)
+    for name, t in (("k", k), ("v", v), ("k_norm", k_norm)):
+        if t is not None and (t.shape != q.shape or t.dtype != q.dtype):
+            raise ValueError(f"{name} must be {tuple(q.shape)} {q.dtype}, got {tuple(t.shape)} {t.dtype}")
+    if cache is not None and v is None:
+        raise ValueError("a cache needs the new v")
+    if k_norm is not None and k_norm.stride(-1) != 1:
+        raise ValueError("k_norm must have unit stride in its last dimension")
+    old = [None, None]
+    for i, c in enumerate(cache or ()):
+        if c.dim() != 4 or c.shape[0] not in (1, B) or tuple(c.shape[1:]) != (H, cached, D) or c.dtype != q.dtype:
+            raise ValueError(f"cache must hold [{B} or 1, {H}, {cached}, {D}] {q.dtype}, got {tuple(c.shape)} {c.dtype}")
+        old[i] = _aligned_rows(_bhsd(c, "cache")).expand(B, H, cached, D)
+    _check_shape(S, shape, chunk_thw)
+    _check_shape(cached + S, kv_shape, chunk_thw)
+    code = _dtype_code(q)
+    q, k = _aligned_rows(q), _aligned_rows(k)
+    v = None if v is None else _aligned_rows(v)
+    weights = _norm_weights((q_weight, k_weight), q)
+    lib = _lib.load()
+    g = _lib.Grid(*(int(x) for x in grid))
+    table = _device_table(lib, D, g, grid, q.device)
+    nb, nk = num_blocks(shape, chunk_thw), num_blocks(kv_shape, chunk_thw)
+    q_out = torch.empty((B, H, S, D), dtype=q.dtype, device=q.device)
+    k_out = torch.empty(full, dtype=q.dtype, device=q.device)
+    v_out = None if v is None else torch.empty(full, dtype=q.dtype, device=q.device)
+    q_blocks = torch.empty((B, H, nb, D), dtype=torch.float32, device=q.device)
+    k_blocks = torch.empty((B, H, nk, D), dtype=torch.float32, device=q.device)
+    none = _lib.Strides(0, 0, D)
+
+    def strides(t):
+        return none if t is None else _strides(t)
+
+    st = lib.lcv_bsa_prepare_qkv(
+        q.data_ptr(), k.data_ptr(), _ptr(v), code, B, H, S, D, _strides(q), _strides(k), strides(v),
+        _ptr(old[0]), _ptr(old[1]), cached, strides(old[0]), strides(old[1]), _ptr(weights[0]), _ptr(weights[1]),
+        float(eps), g, table.data_ptr(), table.numel(), _geom(shape, chunk_thw), _geom(kv_shape, chunk_thw),
+        q_out.data_ptr(), k_out.data_ptr(), _ptr(v_out), _ptr(k_norm), _strides(q_out), _strides(k_out),
+        strides(v_out), strides(k_norm), q_blocks.data_ptr(), k_blocks.data_ptr(), _stream(q),
+    )
+    _lib.check(st, "prepare_qkv")
+    return q_out, k_out, v_out, q_blocks, k_blocks
