@@ -223,6 +223,22 @@ int lcv_bsa_head_rms_norm(const void* x, int dtype, int64_t B, int64_t H,
                           lcv_bsa_strides os, void* stream);
 
 /*
+ * Text cross-attention (attention.py:318-352).  q [B,H,N,D] is normalised per
+ * row as lcv_bsa_head_rms_norm does (weight q_weight [D], eps); item b then
+ * attends to its own text_len[b] >= 1 rows of the packed k, v [H,L,D] (strides
+ * h and s; the items' rows follow one another, their sum is at most L), with
+ * softmax(sm_scale * q.k).  k is normalised already.  text_len is read on the
+ * host.  fp16 / bf16, D in {64, 128}, any N and lengths, sm_scale >= 0, rows
+ * on 16-byte boundaries.  Writes out [B,H,N,D].
+ */
+int lcv_bsa_text_attn(const void* q, const void* k, const void* v, int dtype,
+                      int64_t B, int64_t H, int64_t N, int64_t L, int64_t D,
+                      lcv_bsa_strides qs, lcv_bsa_strides ks,
+                      lcv_bsa_strides vs, const int64_t* text_len,
+                      const void* q_weight, float eps, float sm_scale,
+                      void* out, lcv_bsa_strides os, void* stream);
+
+/*
  * Bytes of workspace lcv_bsa_forward needs: the fp32 pooled means of q and
  * k (2*B*H*nb*D*4 bytes), the fp32 block scores (B*H*nb*nb*4 bytes) and the
  * int32 launch order (B*H*nb*4 bytes), each rounded up to 256 bytes.  Host

@@ -248,6 +248,20 @@ hipError_t launch_head_norm(const void* x, const int64_t* xs, void* out, const i
                             const void* w, int dtype, int B, int N, int H, int D, float eps,
                             hipStream_t stream);
 
+// Text cross-attention of B batch items (at most kTextItems), q rows normalised
+// on the way in: item b's N queries attend to keys start[b] .. start[b] + len[b] - 1
+// (len >= 1) of the packed k / v (sb unused).  fp16 / bf16, D 64 / 128, rows on
+// 16-byte boundaries, scale >= 0, every item's k / v rows within 4 GiB.
+constexpr int kTextItems = 32;
+struct TextAttn {
+  Tensor4 q, k, v, out;
+  const void* q_weight;  // [D] in the dtype
+  int32_t B, H, N;
+  float eps, scale_log2;
+  int32_t start[kTextItems], len[kTextItems];
+};
+hipError_t launch_text_attn(const TextAttn& t, int dtype, int D, hipStream_t stream);
+
 hipError_t launch_token_blocks(const Geom& g, int T, int32_t* out, hipStream_t stream);
 hipError_t launch_pair_mask(const int32_t* idx, int B, int H, int nq, int top_k,
                             const int32_t* token_block, int S, int nkv, uint8_t* mask,

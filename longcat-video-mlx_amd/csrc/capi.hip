@@ -680,6 +680,63 @@ int lcv_bsa_head_rms_norm(const void* x, int dtype, int64_t B, int64_t H, int64_
                        "lcv_bsa_head_rms_norm");
 }
 
+int lcv_bsa_text_attn(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t H,
+                      int64_t N, int64_t L, int64_t D, lcv_bsa_strides qs, lcv_bsa_strides ks,
+                      lcv_bsa_strides vs, const int64_t* text_len, const void* q_weight, float eps,
+                      float sm_scale, void* out, lcv_bsa_strides os, void* stream) {
+  if (!q || !k || !v || !out || !q_weight || !text_len)
+    return fail(LCV_BSA_ERR_INVALID_ARG, "null pointer");
+  if (dtype != LCV_BSA_F16 && dtype != LCV_BSA_BF16)
+    return fail(LCV_BSA_ERR_DTYPE, "text attention takes fp16 or bf16 (got dtype %d)", dtype);
+  if (!(D == 64 || D == 128))
+    return fail(LCV_BSA_ERR_UNSUPPORTED, "text attention needs D in {64, 128}");
+  if (B <= 0 || H <= 0 || N <= 0 || L <= 0 || B > kI32Max || H > kI32Max || N > kI32Max / 2 ||
+      L > kI32Max / 2 || B * H > kI32Max / 4 || B * H * ((N + 127) / 128) > kI32Max / 256)
+    return fail(LCV_BSA_ERR_SHAPE, "B=%lld H=%lld N=%lld L=%lld must be positive and within one launch",
+                (long long)B, (long long)H, (long long)N, (long long)L);
+  if (!std::isfinite(eps) || eps < 0.0f) return fail(LCV_BSA_ERR_INVALID_ARG, "eps must be >= 0");
+  if (!std::isfinite(sm_scale) || sm_scale < 0.0f)
+    return fail(LCV_BSA_ERR_UNSUPPORTED, "text attention needs a finite sm_scale >= 0");
+  int64_t total = 0;
+  for (int64_t b = 0; b < B; ++b) {
+    if (text_len[b] < 1 || text_len[b] > L - total)
+      return fail(LCV_BSA_ERR_SHAPE, "text length %lld of item %lld: each must be >= 1, all within the %lld rows",
+                  (long long)text_len[b], (long long)b, (long long)L);
+    total += text_len[b];
+  }
+  int st = 0;
+  if ((st = check_strides("q", qs, D)) || (st = check_strides("k", ks, D)) ||
+      (st = check_strides("v", vs, D)) || (st = check_strides("out", os, D)))
+    return st;
+  if (!vec_aligned(q, qs, 8) || !vec_aligned(k, ks, 8) || !vec_aligned(v, vs, 8) ||
+      !vec_aligned(out, os, 8) || (uintptr_t)q_weight % 16)
+    return fail(LCV_BSA_ERR_LAYOUT, "rows and weight must start on 16-byte boundaries");
+  if (head_bytes(L, ks.s, D, dtype) > 0xFFFFFFFFull || head_bytes(L, vs.s, D, dtype) > 0xFFFFFFFFull)
+    return fail(LCV_BSA_ERR_LAYOUT, "one head of k or v spans more than 4 GiB");
+  int64_t off = 0;
+  for (int64_t b0 = 0; b0 < B; b0 += lcv::kTextItems) {
+    lcv::TextAttn t{};
+    t.B = (int32_t)std::min<int64_t>(lcv::kTextItems, B - b0);
+    t.H = (int32_t)H;
+    t.N = (int32_t)N;
+    t.q = {(const char*)q + 2 * b0 * qs.b, qs.b, qs.h, qs.s};
+    t.k = {k, 0, ks.h, ks.s};
+    t.v = {v, 0, vs.h, vs.s};
+    t.out = {(char*)out + 2 * b0 * os.b, os.b, os.h, os.s};
+    t.q_weight = q_weight;
+    t.eps = eps;
+    t.scale_log2 = sm_scale * 1.4426950408889634f;
+    for (int i = 0; i < t.B; ++i) {
+      t.start[i] = (int32_t)off;
+      t.len[i] = (int32_t)text_len[b0 + i];
+      off += text_len[b0 + i];
+    }
+    if ((st = launch_status(lcv::launch_text_attn(t, dtype, (int)D, (hipStream_t)stream), "lcv_bsa_text_attn")))
+      return st;
+  }
+  return ok();
+}
+
 int lcv_bsa_token_blocks(lcv_bsa_geom g, int32_t* out, void* stream) {
   if (!out) return fail(LCV_BSA_ERR_INVALID_ARG, "null pointer");
   int64_t nb = 0, bs = 0;

@@ -6,18 +6,21 @@ the cross-attention pre-norm (longcat_video_dit.py:107-136; blocks.py:
 the cross-attention's per-head q / k norms (attention.py:325-326).  Each is
 one pass over HBM through ``liblcv_bsa.so``; each rounds like the
 reference's sequence of fp32 tensor operations followed by a cast.
+``text_attention`` is the cross-attention itself with the q norm inside
+(attention.py:318-352).
 """
 
 from __future__ import annotations
 
-from typing import Optional
+import ctypes
+from typing import Optional, Sequence
 
 import torch
 
 from . import _lib
 from .block_sparse_attention import _dtype_code, _require_device, _stream, _strides
 
-__all__ = ["residual_norm", "swiglu", "head_rms_norm", "plain_tensors"]
+__all__ = ["residual_norm", "swiglu", "head_rms_norm", "text_attention", "plain_tensors"]
 
 
 def plain_tensors(*ts: Optional[torch.Tensor]) -> bool:
@@ -121,4 +124,29 @@ def head_rms_norm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float = 
         x.data_ptr(), _dtype_code(x), B, H, S, D, _strides(x), _ptr(weight), float(eps),
         out.data_ptr(), _strides(out), _stream(x))
     _lib.check(st, "head_rms_norm")
+    return out
+
+
+def text_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, text_len: Sequence[int],
+                   q_weight: torch.Tensor, eps: float, sm_scale: float, out: torch.Tensor) -> torch.Tensor:
+    """``q`` ``[B, H, N, D]`` (normalised here, RMSNorm_FP32) over the packed
+    text ``k`` (normalised), ``v`` ``[H, L, D]``: item b attends to the
+    ``text_len[b]`` rows after those of the items before it.  Writes ``out``
+    ``[B, H, N, D]`` (any strides with dense D)."""
+    _require_device(q, k, v, out)
+    B, H, N, D = q.shape
+    L = k.shape[1]
+    if tuple(k.shape) != (H, L, D) or tuple(v.shape) != (H, L, D) or tuple(out.shape) != (B, H, N, D):
+        raise ValueError(f"k, v must be [{H}, L, {D}] and out {tuple(q.shape)}: got {tuple(k.shape)}, "
+                         f"{tuple(v.shape)}, {tuple(out.shape)}")
+    if len(text_len) != B:
+        raise ValueError(f"{len(text_len)} text lengths for {B} batch items")
+    if not (q.dtype == k.dtype == v.dtype == out.dtype) or any(t.stride(-1) != 1 for t in (q, k, v, out)):
+        raise ValueError("q, k, v, out must share a dtype and have unit stride in their last dimension")
+    weight = _rows(q_weight.to(q.dtype), "q_weight", (D,))
+    st = _lib.load().lcv_bsa_text_attn(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _dtype_code(q), B, H, N, L, D, _strides(q), _strides(k[None]),
+        _strides(v[None]), (ctypes.c_int64 * B)(*text_len), weight.data_ptr(), float(eps), float(sm_scale),
+        out.data_ptr(), _strides(out), _stream(q))
+    _lib.check(st, "text_attention")
     return out

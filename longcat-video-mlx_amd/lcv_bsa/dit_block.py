@@ -24,9 +24,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .attention import BSAAttention, dense_attention, validate_backend
-from .block_ops import head_rms_norm, plain_tensors, residual_norm, swiglu
+from .block_ops import head_rms_norm, plain_tensors, residual_norm, swiglu, text_attention
 from .block_sparse_attention import bsa_attention
-from .block_sparse_attention_hip import bsa_attention_hip
 from .prepare import prepare_qk, prepare_qkv
 from .rope_3d import rope_3d
 from .shape_policy import bsa_geometry
@@ -308,8 +307,8 @@ class MultiHeadCrossAttention(nn.Module):
         self.proj = nn.Linear(dim, dim, **kw)
         self.q_norm = RMSNorm_FP32(self.head_dim, eps=1e-6, **kw)
         self.k_norm = RMSNorm_FP32(self.head_dim, eps=1e-6, **kw)
-        # On the GPU, with 64-aligned token and text lengths: fused norms and
-        # the library's attention kernel (dense over the text blocks).
+        # On the GPU in half precision: k's norm, then q's norm and the attention
+        # over each item's text in one kernel.
         self.fused = True
 
     def forward(self, x: torch.Tensor, cond: torch.Tensor, kv_seqlen: Sequence[int],
@@ -324,42 +323,46 @@ class MultiHeadCrossAttention(nn.Module):
             return torch.cat([out_noise.new_zeros((B, nc, C)), out_noise], dim=1)
         return self._cross(x, cond, kv_seqlen)
 
-    def _cross_fused(self, x, cond, kv_seqlen):
-        """q / k norms in place on the projections' rows, then the library's
-        attention kernel with every text block listed (dense over the text),
-        written in the [B, N, H, D] layout the projection reads."""
-        B, N, C = x.shape
-        H, D = self.num_heads, self.head_dim
-        q = self.q_linear(x).view(B, N, H, D).transpose(1, 2)      # [B, H, N, D] view
-        head_rms_norm(q, self.q_norm.weight, self.q_norm.eps, out=q)
-        kv = self.kv_linear(cond).view(1, -1, 2, H, D)
-        k = kv[:, :, 0].transpose(1, 2)
-        head_rms_norm(k, self.k_norm.weight, self.k_norm.eps, out=k)
-        v = kv[:, :, 1].transpose(1, 2)
-        o = torch.empty((B, N, H, D), dtype=x.dtype, device=x.device)
-        off = 0
-        for b in range(B):
-            n = int(kv_seqlen[b])
-            nk = n // 64
-            idx = torch.arange(nk, dtype=torch.int32, device=x.device).expand(1, H, N // 64, nk).contiguous()
-            bsa_attention_hip(q[b:b + 1], k[:, :, off:off + n], v[:, :, off:off + n], idx, (1, 1, 64),
-                              (1, 1, N), self.scale, out=o[b:b + 1].transpose(1, 2), kv_shape=(1, 1, n))
-            off += n
-        return self.proj(o.view(B, N, C))
+    def _fusible(self, q, kv, lens) -> bool:
+        """Whether the text attention kernel takes these projections: 64-token
+        multiples always; any other lengths where nothing differentiates or
+        traces through the norms and the attention, and the lengths share out
+        text that is there."""
+        if self.head_dim not in (64, 128) or not q.is_cuda or q.dtype not in (torch.float16, torch.bfloat16):
+            return False
+        if q.shape[1] % 64 == 0 and all(n % 64 == 0 for n in lens):
+            return True
+        n = lens[:q.shape[0]]
+        return (len(n) == q.shape[0] and min(n) >= 1 and sum(n) <= kv.shape[1]
+                and plain_tensors(q, kv, self.q_norm.weight, self.k_norm.weight)
+                and q.data_ptr() % 16 == 0 and kv.data_ptr() % 16 == 0)
+
+    def _cross_fused(self, q, kv, lens):
+        """q [B, N, H, D], kv [1, L, 2, H, D]: k's norm, then q's norm and the
+        attention as one kernel over each item's own text, written in the
+        [B, N, H, D] layout the projection reads."""
+        q_weight, k_weight = (w if w.data_ptr() % 16 == 0 else w.clone()
+                              for w in (self.q_norm.weight, self.k_norm.weight))
+        k = head_rms_norm(kv[:, :, 0].transpose(1, 2), k_weight, self.k_norm.eps)[0]
+        o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        text_attention(q.transpose(1, 2), k, kv[0, :, 1].transpose(0, 1), lens[:q.shape[0]], q_weight,
+                       self.q_norm.eps, self.scale, o.transpose(1, 2))
+        return self.proj(o.view(*q.shape[:2], self.dim))
 
     def _cross(self, x: torch.Tensor, cond: torch.Tensor, kv_seqlen: Sequence[int]) -> torch.Tensor:
         B, N, C = x.shape
         H, D = self.num_heads, self.head_dim
-        if (self.fused and x.is_cuda and N % 64 == 0 and all(int(n) % 64 == 0 for n in kv_seqlen)
-                and D in (64, 128) and x.dtype in (torch.float16, torch.bfloat16)):
-            return self._cross_fused(x, cond, kv_seqlen)
-        q = self.q_norm(self.q_linear(x).view(B, N, H, D)).transpose(1, 2).contiguous()
+        lens = [int(n) for n in kv_seqlen]
+        q = self.q_linear(x).view(B, N, H, D)
         kv = self.kv_linear(cond).view(1, -1, 2, H, D)
+        if self.fused and x.is_cuda and x.dtype == q.dtype and self._fusible(q, kv, lens):
+            return self._cross_fused(q, kv, lens)
+        q = self.q_norm(q).transpose(1, 2).contiguous()
         k = self.k_norm(kv[:, :, 0]).transpose(1, 2).contiguous()
         v = kv[:, :, 1].transpose(1, 2).contiguous()
         outs, off = [], 0
         for b in range(B):
-            n = int(kv_seqlen[b])
+            n = lens[b]
             outs.append(dense_attention(q[b:b + 1], k[..., off:off + n, :], v[..., off:off + n, :], self.scale))
             off += n
         o = torch.cat(outs, 0) if B > 1 else outs[0]
