@@ -263,6 +263,24 @@ int lcv_bsa_forward(const void* q, const void* k, const void* v, int dtype,
                     int32_t* idx, void* out, lcv_bsa_strides os,
                     void* stream);
 
+/*
+ * lcv_bsa_forward with S_q != S_k: q and out in grid gq (nq blocks), k and v in
+ * grid gk (nk blocks), the same voxel; each q-block keeps top_k of the nk
+ * k-blocks.  qbar [B,H,nq,D], kbar [B,H,nk,D]: the fp32 block means where the
+ * caller has them (lcv_bsa_prepare_qk), else both null.  The workspace
+ * (256-byte aligned) holds the means, the scores and the launch order.
+ */
+size_t lcv_bsa_forward_kv_workspace_bytes(int64_t B, int64_t H, int64_t nq,
+                                          int64_t nk, int64_t D);
+int lcv_bsa_forward_kv(const void* q, const void* k, const void* v, int dtype,
+                       int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,
+                       lcv_bsa_strides qs, lcv_bsa_strides ks,
+                       lcv_bsa_strides vs, const float* qbar,
+                       const float* kbar, int64_t top_k, float sm_scale,
+                       lcv_bsa_geom gq, lcv_bsa_geom gk, void* workspace,
+                       size_t workspace_bytes, int32_t* idx, void* out,
+                       lcv_bsa_strides os, void* stream);
+
 /* Bytes of device scratch lcv_bsa_forward_noalloc holds per GPU. */
 #define LCV_BSA_NOALLOC_SCRATCH_BYTES ((size_t)1 << 20)
 

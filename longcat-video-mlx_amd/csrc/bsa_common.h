@@ -159,8 +159,9 @@ struct Tensor4 {
   int64_t sb, sh, ss;  // element strides; D axis dense
 };
 
+// One or two tensors, tensor t of nb[t] blocks in geometry g[t] (the same voxel).
 hipError_t launch_pool(const Tensor4* xs, int n_tensors, int dtype, int B, int H,
-                       int D, int nb, int bs, const Geom& g, float* const* outs,
+                       int D, const int* nb, int bs, const Geom* g, float* const* outs,
                        hipStream_t stream);
 
 hipError_t launch_scores(const float* qbar, const float* kbar, int B, int H, int nq,
@@ -170,6 +171,8 @@ hipError_t launch_topk(const float* score, int B, int H, int nq, int nk, int top
 hipError_t launch_select(const float* qbar, const float* kbar, int B, int H, int nq,
                          int nk, int D, int top_k, int32_t* idx, hipStream_t stream);
 bool select_supported(int nk, int D);
+// Whether the fused select beats score GEMM + top-k.
+bool select_short(int BH, int nq, int nk);
 
 struct AttnParams {
   const void* q;
@@ -207,6 +210,8 @@ bool attn_uses_mfma(int dtype, int D);
 hipError_t launch_schedule(const int32_t* idx, int BH, int nq, int nk, int top_k, int32_t* order,
                            hipStream_t stream);
 bool schedule_supported(int nq, int nk);
+// Whether the launch order saves the attention more than its sort costs.
+bool schedule_pays(int nk);
 
 // Fused RMSNorm + 3D RoPE + block means of q and k (fp16/bf16, D 64/128).
 // The RoPE table holds cos and sin per axis: [rT*dt/2 | rT*dt/2 | rH*dh/2 |

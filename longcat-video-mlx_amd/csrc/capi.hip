@@ -214,8 +214,10 @@ int lcv_bsa_pool(const void* x, int dtype, int64_t B, int64_t H, int64_t S, int6
   if ((st = check_strides("x", xs, D))) return st;
   const lcv::Tensor4 t{x, xs.b, xs.h, xs.s};
   float* outs[1] = {out};
-  return launch_status(lcv::launch_pool(&t, 1, dtype, (int)B, (int)H, (int)D, (int)nb, (int)bs,
-                                        lcv::make_geom(g), outs, (hipStream_t)stream),
+  const int n = (int)nb;
+  const lcv::Geom geom = lcv::make_geom(g);
+  return launch_status(lcv::launch_pool(&t, 1, dtype, (int)B, (int)H, (int)D, &n, (int)bs, &geom, outs,
+                                        (hipStream_t)stream),
                        "lcv_bsa_pool");
 }
 
@@ -308,8 +310,8 @@ size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 size_t pooled_bytes(int64_t B, int64_t H, int64_t nb, int64_t D) {
   return align256((size_t)B * H * nb * D * sizeof(float));
 }
-size_t score_bytes(int64_t B, int64_t H, int64_t nb) {
-  return align256((size_t)B * H * nb * nb * sizeof(float));
+size_t score_bytes(int64_t B, int64_t H, int64_t nb, int64_t nk) {
+  return align256((size_t)B * H * nb * nk * sizeof(float));
 }
 }  // namespace
 
@@ -317,7 +319,7 @@ extern "C" {
 
 size_t lcv_bsa_forward_workspace_bytes(int64_t B, int64_t H, int64_t nb, int64_t D) {
   if (B <= 0 || H <= 0 || nb <= 0 || D <= 0) return 0;
-  return 2 * pooled_bytes(B, H, nb, D) + score_bytes(B, H, nb) +
+  return 2 * pooled_bytes(B, H, nb, D) + score_bytes(B, H, nb, nb) +
          align256((size_t)B * H * nb * sizeof(int32_t));
 }
 
@@ -342,61 +344,65 @@ int check_forward_args(const void* q, const void* k, const void* v, int dtype, i
   return check_route(B, H, *nb, *nb, D, true);
 }
 
-// pool -> routing -> schedule -> attention on validated arguments.  With a
-// score buffer the routing runs as the score GEMM (each staged key chunk
-// shared by 64 rows) plus the per-row top-k, score_bh (b, h) slices at a
-// time (all of them when the buffer holds B*H slices); without one, as the
-// fused select kernel that keeps the scores on chip.  All give the same
-// routing.
+// pool -> routing -> schedule -> attention on validated arguments (qbar and
+// kbar hold the means already when `pooled`).  Small grids route in one kernel
+// that keeps the scores on chip.  Otherwise, with a score buffer, the routing
+// runs as the score GEMM (each staged key chunk shared by 64 rows) plus the
+// per-row top-k, score_bh (b, h) slices at a time (all of them when the buffer
+// holds B*H slices); without one, as the fused kernel at any size.  All give
+// the same routing.
 int run_forward(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t H,
-                int64_t S, int64_t D, const lcv_bsa_strides& qs, const lcv_bsa_strides& ks,
+                int64_t Sk, int64_t D, const lcv_bsa_strides& qs, const lcv_bsa_strides& ks,
                 const lcv_bsa_strides& vs, int64_t top_k, float sm_scale, const lcv_bsa_geom& g,
-                int64_t nb, int64_t bs, float* qbar, float* kbar, float* score, int64_t score_bh,
-                int32_t* order, int32_t* idx, void* out, const lcv_bsa_strides& os, hipStream_t s,
-                const char* name) {
+                const lcv_bsa_geom& gk, int64_t nb, int64_t nk, int64_t bs, bool pooled, float* qbar,
+                float* kbar, float* score, int64_t score_bh, int32_t* order, int32_t* idx, void* out,
+                const lcv_bsa_strides& os, hipStream_t s, const char* name) {
   char what[96];
-  const lcv::Tensor4 ts[2] = {{q, qs.b, qs.h, qs.s}, {k, ks.b, ks.h, ks.s}};
-  float* outs[2] = {qbar, kbar};
-  const lcv::Geom gg = lcv::make_geom(g);
-  snprintf(what, sizeof(what), "%s(pool)", name);
-  int st = launch_status(lcv::launch_pool(ts, 2, dtype, (int)B, (int)H, (int)D, (int)nb, (int)bs,
-                                          gg, outs, s),
-                         what);
-  if (st) return st;
-  if (score) {
+  int st = LCV_BSA_OK;
+  if (!pooled) {
+    const lcv::Tensor4 ts[2] = {{q, qs.b, qs.h, qs.s}, {k, ks.b, ks.h, ks.s}};
+    float* outs[2] = {qbar, kbar};
+    const int nbs[2] = {(int)nb, (int)nk};
+    const lcv::Geom geoms[2] = {lcv::make_geom(g), lcv::make_geom(gk)};
+    snprintf(what, sizeof(what), "%s(pool)", name);
+    st = launch_status(lcv::launch_pool(ts, 2, dtype, (int)B, (int)H, (int)D, nbs, (int)bs, geoms, outs, s),
+                       what);
+    if (st) return st;
+  }
+  if (score && !lcv::select_short((int)(B * H), (int)nb, (int)nk)) {
     // Slices [c0, c0 + n) of the B*H (b, h) pairs; the scores of one slice
     // are read by its top-k before the next slice's GEMM rewrites them (one
     // stream).
     for (int64_t c0 = 0; c0 < B * H && !st; c0 += score_bh) {
       const int64_t n = B * H - c0 < score_bh ? B * H - c0 : score_bh;
       snprintf(what, sizeof(what), "%s(scores)", name);
-      st = launch_status(lcv::launch_scores(qbar + c0 * nb * D, kbar + c0 * nb * D, 1, (int)n,
-                                            (int)nb, (int)nb, (int)D, score, s),
+      st = launch_status(lcv::launch_scores(qbar + c0 * nb * D, kbar + c0 * nk * D, 1, (int)n,
+                                            (int)nb, (int)nk, (int)D, score, s),
                          what);
       if (st) return st;
       snprintf(what, sizeof(what), "%s(top-k)", name);
-      st = launch_status(lcv::launch_topk(score, 1, (int)n, (int)nb, (int)nb, (int)top_k,
+      st = launch_status(lcv::launch_topk(score, 1, (int)n, (int)nb, (int)nk, (int)top_k,
                                           idx + c0 * nb * top_k, s),
                          what);
     }
   } else {
     snprintf(what, sizeof(what), "%s(select)", name);
-    st = launch_status(lcv::launch_select(qbar, kbar, (int)B, (int)H, (int)nb, (int)nb, (int)D,
+    st = launch_status(lcv::launch_select(qbar, kbar, (int)B, (int)H, (int)nb, (int)nk, (int)D,
                                           (int)top_k, idx, s),
                        what);
   }
   if (st) return st;
-  const bool sched = lcv::schedule_supported((int)nb, (int)nb);
+  const bool sched = lcv::schedule_supported((int)nb, (int)nk) && lcv::schedule_pays((int)nk);
   if (sched) {
     snprintf(what, sizeof(what), "%s(schedule)", name);
-    st = launch_status(lcv::launch_schedule(idx, (int)(B * H), (int)nb, (int)nb, (int)top_k, order,
+    st = launch_status(lcv::launch_schedule(idx, (int)(B * H), (int)nb, (int)nk, (int)top_k, order,
                                             s),
                        what);
     if (st) return st;
   }
   const lcv::AttnParams p = make_attn_params(q, k, v, out, qs, ks, vs, os, idx,
-                                             sched ? order : nullptr, B, H, S, D, dtype, nb, nb,
-                                             top_k, sm_scale, g, g);
+                                             sched ? order : nullptr, B, H, Sk, D, dtype, nb, nk,
+                                             top_k, sm_scale, g, gk);
   snprintf(what, sizeof(what), "%s(attn)", name);
   return launch_status(lcv::launch_attn(p, dtype, (int)D, s), what);
 }
@@ -524,11 +530,49 @@ int lcv_bsa_forward(const void* q, const void* k, const void* v, int dtype, int6
                 workspace_bytes);
   const size_t pb = pooled_bytes(B, H, nb, D);
   char* ws = reinterpret_cast<char*>(workspace);
-  return run_forward(q, k, v, dtype, B, H, S, D, qs, ks, vs, top_k, sm_scale, g, nb, bs,
-                     reinterpret_cast<float*>(ws), reinterpret_cast<float*>(ws + pb),
+  return run_forward(q, k, v, dtype, B, H, S, D, qs, ks, vs, top_k, sm_scale, g, g, nb, nb, bs,
+                     false, reinterpret_cast<float*>(ws), reinterpret_cast<float*>(ws + pb),
                      reinterpret_cast<float*>(ws + 2 * pb), B * H,
-                     reinterpret_cast<int32_t*>(ws + 2 * pb + score_bytes(B, H, nb)), idx, out, os,
+                     reinterpret_cast<int32_t*>(ws + 2 * pb + score_bytes(B, H, nb, nb)), idx, out, os,
                      (hipStream_t)stream, "lcv_bsa_forward");
+}
+
+size_t lcv_bsa_forward_kv_workspace_bytes(int64_t B, int64_t H, int64_t nq, int64_t nk, int64_t D) {
+  if (B <= 0 || H <= 0 || nq <= 0 || nk <= 0 || D <= 0) return 0;
+  return pooled_bytes(B, H, nq, D) + pooled_bytes(B, H, nk, D) + score_bytes(B, H, nq, nk) +
+         align256((size_t)B * H * nq * sizeof(int32_t));
+}
+
+int lcv_bsa_forward_kv(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t H,
+                       int64_t Sq, int64_t Sk, int64_t D, lcv_bsa_strides qs, lcv_bsa_strides ks,
+                       lcv_bsa_strides vs, const float* qbar, const float* kbar, int64_t top_k,
+                       float sm_scale, lcv_bsa_geom gq, lcv_bsa_geom gk, void* workspace,
+                       size_t workspace_bytes, int32_t* idx, void* out, lcv_bsa_strides os,
+                       void* stream) {
+  int64_t nq = 0, nk = 0, bs = 0;
+  int st = check_attn_args(q, k, v, out, dtype, B, H, Sq, Sk, D, qs, ks, vs, os, top_k, sm_scale, gq,
+                           gk, &nq, &nk, &bs);
+  if (st) return st;
+  if (!idx) return fail(LCV_BSA_ERR_INVALID_ARG, "null idx pointer");
+  if ((!qbar) != (!kbar)) return fail(LCV_BSA_ERR_INVALID_ARG, "qbar and kbar go together");
+  if (top_k > nk)
+    return fail(LCV_BSA_ERR_INVALID_ARG, "top_k=%lld exceeds num_blocks=%lld", (long long)top_k,
+                (long long)nk);
+  if ((st = check_route(B, H, nq, nk, D, true))) return st;
+  const size_t need = lcv_bsa_forward_kv_workspace_bytes(B, H, nq, nk, D);
+  if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255u))
+    return fail(LCV_BSA_ERR_INVALID_ARG,
+                "workspace must be 256-byte aligned and hold %zu bytes (got %zu)", need,
+                workspace_bytes);
+  char* ws = reinterpret_cast<char*>(workspace);
+  float* qb = reinterpret_cast<float*>(ws);
+  float* kb = reinterpret_cast<float*>(ws + pooled_bytes(B, H, nq, D));
+  float* score = reinterpret_cast<float*>(ws + pooled_bytes(B, H, nq, D) + pooled_bytes(B, H, nk, D));
+  int32_t* order = reinterpret_cast<int32_t*>(reinterpret_cast<char*>(score) + score_bytes(B, H, nq, nk));
+  const bool pooled = qbar != nullptr;
+  return run_forward(q, k, v, dtype, B, H, Sk, D, qs, ks, vs, top_k, sm_scale, gq, gk, nq, nk, bs, pooled,
+                     pooled ? const_cast<float*>(qbar) : qb, pooled ? const_cast<float*>(kbar) : kb, score,
+                     B * H, order, idx, out, os, (hipStream_t)stream, "lcv_bsa_forward_kv");
 }
 
 int lcv_bsa_forward_noalloc(const void* q, const void* k, const void* v, int dtype, int64_t B,
@@ -594,8 +638,8 @@ int lcv_bsa_forward_noalloc(const void* q, const void* k, const void* v, int dty
     return fail(LCV_BSA_ERR_LAUNCH, "lcv_bsa_forward_noalloc: hipStreamWaitEvent: %s",
                 hipGetErrorString(e));
   char* stage = reinterpret_cast<char*>(stage_addr);
-  st = run_forward(q, k, v, dtype, B, H, S, D, qs, ks, vs, top_k, sm_scale, g, nb, bs,
-                   reinterpret_cast<float*>(stage), reinterpret_cast<float*>(stage + pb),
+  st = run_forward(q, k, v, dtype, B, H, S, D, qs, ks, vs, top_k, sm_scale, g, g, nb, nb, bs,
+                   false, reinterpret_cast<float*>(stage), reinterpret_cast<float*>(stage + pb),
                    sliced ? reinterpret_cast<float*>(stage + 2 * pb) : nullptr, score_bh,
                    reinterpret_cast<int32_t*>(d->scratch), idx, out, os, s,
                    "lcv_bsa_forward_noalloc");

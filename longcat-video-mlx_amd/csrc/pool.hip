@@ -62,40 +62,46 @@ constexpr int kBatch = 8;       // row loads in flight per lane
 struct PoolArgs {
   Tensor4 x[2];
   float* out[2];
-  int32_t B, H, D, nb, bs;
-  int32_t items_per_tensor;
+  int32_t B, H, D, bs;
+  int32_t nb[2];
+  int32_t items0;  // blocks of the first tensor
   int32_t total_items;
-  Geom g;
+  Geom g[2];
 };
 
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void pool_kernel(PoolArgs a) {
   __shared__ float part[kWavesPerWg][64 * VEC];
-  __shared__ int32_t row_off[kRowTable];
+  __shared__ int32_t row_table[2][kRowTable];
   // Token offset of each voxel row from the block's first token: the same
-  // for every block, so computed once per workgroup.
+  // for every block of a tensor, so computed once per workgroup.
   const bool table = a.bs <= kRowTable;
   if (table)
-    for (int r = threadIdx.x; r < a.bs; r += blockDim.x) row_off[r] = voxel_row_offset(a.g, r);
+    for (int r = threadIdx.x; r < a.bs; r += blockDim.x) {
+      row_table[0][r] = voxel_row_offset(a.g[0], r);
+      row_table[1][r] = voxel_row_offset(a.g[1], r);
+    }
   __syncthreads();
-  const int wave = threadIdx.x / 64;
+  const int wave = uniform_i32(threadIdx.x / 64);
   const int lane = threadIdx.x % 64;
   const int item_raw = blockIdx.x * kWavesPerWg + wave;
   // Waves past the end still take part in the barriers below.
   const bool valid = item_raw < a.total_items;
   const int item = valid ? item_raw : 0;
 
-  const int t = item / a.items_per_tensor;
-  const int rem = item - t * a.items_per_tensor;
-  const int bh = rem / a.nb;
-  const int n = rem - bh * a.nb;
+  const int t = item >= a.items0 ? 1 : 0;
+  const int rem = item - t * a.items0;
+  const int nb = a.nb[t];
+  const int bh = rem / nb;
+  const int n = rem - bh * nb;
+  const int32_t* row_off = row_table[t];
   const int b = bh / a.H;
   const int h = bh - b * a.H;
 
   const Tensor4 x = a.x[t];
   const T* base = reinterpret_cast<const T*>(x.ptr) + (int64_t)b * x.sb + (int64_t)h * x.sh;
-  const int32_t tok0 = block_base_token(a.g, n);
-  float* out = a.out[t] + ((int64_t)bh * a.nb + n) * a.D;
+  const int32_t tok0 = block_base_token(a.g[t], n);
+  float* out = a.out[t] + ((int64_t)bh * nb + n) * a.D;
   const int DC = a.D / VEC;  // chunks per row
   const float inv_bs = 1.0f / (float)a.bs;
 
@@ -126,7 +132,7 @@ __global__ __launch_bounds__(256) void pool_kernel(PoolArgs a) {
         }
       }
       for (; r < a.bs; r += P)
-        L::add(L::load(col + (int64_t)(tok0 + voxel_row_offset(a.g, r)) * x.ss), acc);
+        L::add(L::load(col + (int64_t)(tok0 + voxel_row_offset(a.g[t], r)) * x.ss), acc);
     }
     // Combine the P partial sums of each column chunk in phase order.
 #pragma unroll
@@ -155,21 +161,22 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 }  // namespace
 
 hipError_t launch_pool(const Tensor4* xs, int n_tensors, int dtype, int B, int H, int D,
-                       int nb, int bs, const Geom& g, float* const* outs,
+                       const int* nb, int bs, const Geom* g, float* const* outs,
                        hipStream_t stream) {
   PoolArgs a{};
-  for (int t = 0; t < n_tensors; ++t) {
-    a.x[t] = xs[t];
-    a.out[t] = outs[t];
+  for (int t = 0; t < 2; ++t) {
+    const int u = t < n_tensors ? t : 0;
+    a.x[t] = xs[u];
+    a.out[t] = outs[u];
+    a.nb[t] = nb[u];
+    a.g[t] = g[u];
   }
   a.B = B;
   a.H = H;
   a.D = D;
-  a.nb = nb;
   a.bs = bs;
-  a.items_per_tensor = B * H * nb;
-  a.total_items = a.items_per_tensor * n_tensors;
-  a.g = g;
+  a.items0 = B * H * nb[0];
+  a.total_items = a.items0 + (n_tensors == 2 ? B * H * nb[1] : 0);
 
   const int elem = dtype == LCV_BSA_F32 ? 4 : 2;
   const int vec = 16 / elem;

@@ -1,4 +1,5 @@
-// Launch order of the q-blocks of each head for the attention kernel.
+// Launch order of the q-blocks of each head for the attention kernel, for heads
+// of more than 320 K/V blocks (schedule_pays).
 //
 // Any order gives the same results up to fp32 rounding: each q-block is
 // computed by one workgroup from its own routing list, and its launch slot
@@ -155,6 +156,14 @@ __global__ __launch_bounds__(256) void schedule_rank_small_kernel(const int32_t*
 bool schedule_supported(int nq, int nk) {
   return nq >= 1 && nq <= kMaxSched && nk >= 1 && nk <= kMaxKvBlocks;
 }
+
+// The order groups q-blocks that read the same K/V blocks: it pays once a head's
+// blocks outgrow what the resident workgroups share anyway.  Whole forward with one
+// sixteenth of the blocks kept, without against with the order: 92.4 / 96.7 us at 32
+// heads x 90 blocks of 64 x 128 fp16, 319.6 / 324.6 us at 225, 531 / 541 us at 312, then
+// 1,034 / 1,027 us at 450 and 306 / 297 us at 2 heads x 900 (D = 64: 311 / 315 us at
+// 320, equal at 450 to 900; fp32: 316 / 320 us at 8 heads x 195 blocks).
+bool schedule_pays(int nk) { return nk > 320; }
 
 hipError_t launch_schedule(const int32_t* idx, int BH, int nq, int nk, int top_k, int32_t* order,
                            hipStream_t stream) {

@@ -497,15 +497,14 @@ __device__ __forceinline__ bool load_row_pieces(const float* base, int row0, int
   return __ballot(!fin) != 0;
 }
 
-// Fused routing for head dims 64 and 128: one workgroup = 16 q-block rows of
-// one (b, h) (the top half of a 32-row MFMA block; the bottom half is zero
-// and discarded); wave w computes the 32-key score tiles w, w + 4, ..., its
-// key operands read from global memory and split in registers.  The 16 x nk
-// score rows are gathered in LDS and each wave runs wave_topk on four of
+// Fused routing for head dims 64 and 128: one workgroup = QR q-block rows of
+// one (b, h) (the first of a 32-row MFMA block; the other rows are zero
+// and discarded); wave w of W computes the 32-key score tiles w, w + W, ..., its
+// key operands read from global memory and split in registers.  The QR x nk
+// score rows are gathered in LDS and each wave runs wave_topk on QR / W of
 // them: routing without a score buffer.
-template <int NPER, int D>
-__global__ __launch_bounds__(256) void select_mfma_kernel(RouteArgs a) {
-  constexpr int QR = 16;
+template <int NPER, int D, int QR, int W>
+__global__ __launch_bounds__(64 * W) void select_mfma_kernel(RouteArgs a) {
   constexpr int KST = D / 16;               // k-steps of 16 dims
   constexpr int LDSW = NPER * 64 + 4;       // score row stride (floats)
   // Row stride: the scores, or the top-k buffer the row turns into (2 CAP words).
@@ -524,7 +523,7 @@ __global__ __launch_bounds__(256) void select_mfma_kernel(RouteArgs a) {
   bf16x8 pa[KST][3];
   const bool a_bad = load_row_pieces<KST>(qb, row0, a.nq, D, QR, pa);
   const int ntiles = (a.nk + 31) / 32;
-  for (int t = wave; t < ntiles; t += 4) {
+  for (int t = wave; t < ntiles; t += W) {
     const int key = 32 * t + c;
     f32x16 acc;
 #pragma unroll
@@ -550,14 +549,14 @@ __global__ __launch_bounds__(256) void select_mfma_kernel(RouteArgs a) {
       else
         tile_step(pa[s], pb, acc);
     }
-    // Rows 8 (i / 4) + 4 g + i % 4 of the tile; i < 8 are the 16 live rows.
+    // Rows 8 (i / 4) + 4 g + i % 4 of the tile; i < QR / 2 are the live rows.
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < QR / 2; ++i)
       srow[(8 * (i / 4) + 4 * g + i % 4) * RSW + 32 * t + c] = acc[i];
   }
   __syncthreads();
 #pragma unroll 1
-  for (int r = wave; r < QR; r += 4) {
+  for (int r = wave; r < QR; r += W) {
     const int row = row0 + r;
     if (row >= a.nq) break;  // wave-uniform; rows only grow
     float sc[NPER];
@@ -730,12 +729,18 @@ hipError_t launch_route_n(RouteArgs a, int BH, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <int NPER, int D>
-hipError_t launch_select_mfma_n(RouteArgs a, int BH, hipStream_t stream) {
-  a.tiles_per_bh = (a.nq + 15) / 16;
-  hipLaunchKernelGGL((select_mfma_kernel<NPER, D>), dim3(BH * a.tiles_per_bh), dim3(256), 0,
+template <int NPER, int D, int QR, int W>
+hipError_t launch_select_tile(RouteArgs a, int BH, hipStream_t stream) {
+  a.tiles_per_bh = (a.nq + QR - 1) / QR;
+  hipLaunchKernelGGL((select_mfma_kernel<NPER, D, QR, W>), dim3(BH * a.tiles_per_bh), dim3(64 * W), 0,
                      stream, a);
   return hipGetLastError();
+}
+
+template <int NPER, int D>
+hipError_t launch_select_mfma_n(RouteArgs a, int BH, hipStream_t stream) {
+  if (select_short(BH, a.nq, a.nk)) return launch_select_tile<NPER, D, 8, 8>(a, BH, stream);
+  return launch_select_tile<NPER, D, 16, 4>(a, BH, stream);
 }
 
 template <int D>
@@ -773,6 +778,14 @@ hipError_t launch_route(RouteArgs a, int BH, hipStream_t stream) {
 }
 
 }  // namespace
+
+// One workgroup of 8 rows and 8 waves per CU at most, and one 32-key tile per
+// wave at most: routing is then one chain of loads, 48 MFMAs and a top-k, and one
+// launch instead of two.  Whole forward against scores + top-k, D = 128, fp16: 23.4
+// against 25.1 us at 2 heads x 32 blocks, 34.2 / 35.8 us at 8 x 64, 119.4 / 122.7 us
+// at 8 x 256; beyond the line 168.5 / 167.8 us at 5 x 400, 363 / 351 us at 2 x 900,
+// 114 / 106 us at 32 x 100.
+bool select_short(int BH, int nq, int nk) { return nk <= 256 && (int64_t)BH * ((nq + 7) / 8) <= 256; }
 
 bool select_supported(int nk, int D) {
   return nk >= 1 && nk <= kMaxPer * 64 && D >= 4 && D <= kMaxD && D % 4 == 0;

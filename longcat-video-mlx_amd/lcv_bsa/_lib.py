@@ -81,6 +81,10 @@ _SIGNATURES = {
     "lcv_bsa_forward": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64,
                                 c_int64, Strides, Strides, Strides, c_int64, c_float, Geom,
                                 c_void_p, c_size_t, c_void_p, c_void_p, Strides, c_void_p]),
+    "lcv_bsa_forward_kv_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64, c_int64, c_int64]),
+    "lcv_bsa_forward_kv": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64,
+                                   c_int64, Strides, Strides, Strides, c_void_p, c_void_p, c_int64, c_float,
+                                   Geom, Geom, c_void_p, c_size_t, c_void_p, c_void_p, Strides, c_void_p]),
     "lcv_bsa_forward_noalloc": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64,
                                         c_int64, Strides, Strides, Strides, c_int64, c_float, Geom,
                                         c_void_p, c_void_p, Strides, c_void_p]),

@@ -50,7 +50,7 @@ _DTYPES = {torch.float16: _lib.F16, torch.bfloat16: _lib.BF16, torch.float32: _l
 # ---------------------------------------------------------------------------
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 class BSADeviceError(RuntimeError):
@@ -82,7 +82,7 @@ def _bhsd(t: torch.Tensor, name: str) -> torch.Tensor:
     """A [B, H, S, D] view whose D axis is dense (copies only when it isn't)."""
     if t.dim() != 4:
         raise ValueError(f"{name} must be [B, H, S, D], got shape {tuple(t.shape)}")
-    if t.stride(3) != 1 or any(s < 0 for s in t.stride()):
+    if t.stride(3) != 1:
         t = t.contiguous()
     return t
 
@@ -90,7 +90,8 @@ def _bhsd(t: torch.Tensor, name: str) -> torch.Tensor:
 def _aligned_rows(t: torch.Tensor) -> torch.Tensor:
     """Rows 16-byte aligned (what the MFMA kernel loads); copy otherwise."""
     vec = 16 // t.element_size()
-    if t.data_ptr() % 16 or any(s % vec for s in t.stride()[:3]):
+    sb, sh, ss, _ = t.stride()
+    if t.data_ptr() % 16 or (sb | sh | ss) % vec:
         t = t.contiguous()
         if t.data_ptr() % 16:
             t = t.clone()
@@ -311,25 +312,19 @@ def bsa_attention(
     kk = num_selected_blocks(nk, sparsity) if top_k is None else int(top_k)
     if not 1 <= kk <= nk:
         raise ValueError(f"top_k={kk} must be in [1, {nk}]")
-    if block_means is not None or kv_shape is not None:
-        from .block_sparse_attention_hip import bsa_attention_hip
-
-        if kv_shape is not None:
-            if not (k.shape == v.shape and k.shape[:2] == q.shape[:2] and k.shape[3] == D):
-                raise ValueError(f"k, v must be [B, H, S_k, D] matching q {tuple(q.shape)}: "
-                                 f"got {tuple(k.shape)}, {tuple(v.shape)}")
-            _check_shape(k.shape[2], kv_shape, chunk_thw)
-        if block_means is not None:
-            qb, kb = block_means
-            for name, t, n in (("q_blocks", qb, nb), ("k_blocks", kb, nk)):
-                if tuple(t.shape) != (B, H, n, D) or t.dtype != torch.float32:
-                    raise ValueError(f"{name} must be fp32 [{B}, {H}, {n}, {D}], got {tuple(t.shape)} {t.dtype}")
-        else:
-            qb = mean_pool_blocks_3d(q, shape, chunk_thw)
-            kb = mean_pool_blocks_3d(k, kv_shape, chunk_thw)
-        idx = select_block_indices(qb, kb, kk)
-        out = bsa_attention_hip(q, k, v, idx, chunk_thw, shape, sm_scale, out=out, kv_shape=kv_shape)
-        return (out, idx) if return_indices else out
+    if kv_shape is not None:
+        if not (k.shape == v.shape and k.shape[:2] == q.shape[:2] and k.shape[3] == D):
+            raise ValueError(f"k, v must be [B, H, S_k, D] matching q {tuple(q.shape)}: "
+                             f"got {tuple(k.shape)}, {tuple(v.shape)}")
+        _check_shape(k.shape[2], kv_shape, chunk_thw)
+    qb = kb = None
+    if block_means is not None:
+        qb, kb = block_means
+        for name, t, n in (("q_blocks", qb, nb), ("k_blocks", kb, nk)):
+            if tuple(t.shape) != (B, H, n, D) or t.dtype != torch.float32:
+                raise ValueError(f"{name} must be fp32 [{B}, {H}, {n}, {D}], got {tuple(t.shape)} {t.dtype}")
+        _require_device(q, qb, kb)
+        qb, kb = qb.contiguous(), kb.contiguous()
     code = _dtype_code(q)
     if code != _lib.F32:
         q, k, v = _aligned_rows(q), _aligned_rows(k), _aligned_rows(v)
@@ -338,13 +333,15 @@ def bsa_attention(
 
     out = _output(out, q)
     idx = torch.empty((B, H, nb, kk), dtype=torch.int32, device=q.device)
-    ws_bytes = lib.lcv_bsa_forward_workspace_bytes(B, H, nb, D)
+    geom = _geom(shape, chunk_thw)
+    geom_kv = geom if kv_shape is None else _geom(kv_shape, chunk_thw)
+    ws_bytes = lib.lcv_bsa_forward_kv_workspace_bytes(B, H, nb, nk, D)
     ws = torch.empty((ws_bytes + 255,), dtype=torch.uint8, device=q.device)
     ws_ptr = (ws.data_ptr() + 255) // 256 * 256
-    st = lib.lcv_bsa_forward(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), code, B, H, S, D,
-        _strides(q), _strides(k), _strides(v), kk, float(sm_scale), _geom(shape, chunk_thw),
-        ws_ptr, ws_bytes, idx.data_ptr(), out.data_ptr(), _strides(out), _stream(q),
+    st = lib.lcv_bsa_forward_kv(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), code, B, H, S, k.shape[2], D, _strides(q), _strides(k), _strides(v),
+        None if qb is None else qb.data_ptr(), None if kb is None else kb.data_ptr(), kk, float(sm_scale), geom,
+        geom_kv, ws_ptr, ws_bytes, idx.data_ptr(), out.data_ptr(), _strides(out), _stream(q),
     )
     _lib.check(st, "bsa_attention")
     return (out, idx) if return_indices else out
