@@ -210,6 +210,17 @@ int lcv_bsa_block_swiglu(const void* h13, int dtype, int64_t rows,
                          int64_t hidden, void* out, void* stream);
 
 /*
+ * AdaLN modulation (longcat_video_dit.py:80-138) in fp32: out[j,r,c] =
+ * bias[j*C + c] + sum_k silu(t[r,k]) * weight[j*C + c, k] for fp32 t [R,K] and
+ * half-precision weight [chunks*C, K] and bias, written as fp32
+ * [chunks, R, C].  K % 8 == 0, K <= 1024, C % 8 == 0; t and weight 16-byte
+ * aligned.
+ */
+int lcv_bsa_adaln(const float* t, const void* weight, const void* bias,
+                  int dtype, int64_t R, int64_t K, int64_t chunks, int64_t C,
+                  float* out, void* stream);
+
+/*
  * Per-head RMSNorm_FP32 (blocks.py:55-72) of a [B,H,S,D] view into another
  * [B,H,S,D] view (strides in elements, any layout with dense D):
  *   out = round(round(x * rsqrt(mean(x^2) + eps)) * weight).

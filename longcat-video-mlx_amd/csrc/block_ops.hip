@@ -7,6 +7,8 @@
 //    (longcat_video_dit.py:107-136 with blocks.py:79-119);
 //  * SwiGLU gate: silu(a) * b over the two halves of the fused w1 / w3
 //    projection (blocks.py:50-51);
+//  * AdaLN modulation: silu(t) W^T + b in fp32 from the half-precision weight,
+//    written chunk by chunk (longcat_video_dit.py:80-138);
 //  * per-head RMSNorm_FP32 (blocks.py:55-72) from one layout to another, for
 //    the cross-attention's q and k (attention.py:325-326).
 //
@@ -213,6 +215,108 @@ __global__ __launch_bounds__(256) void head_norm_kernel(HeadNormArgs p) {
   if (ok) store8(reinterpret_cast<T*>(p.out) + b * p.o_sb + n * p.o_sn + h * p.o_sh + 8 * c, y);
 }
 
+// out[j][r][c] = b[j C + c] + sum_k silu(t[r][k]) W[j C + c][k], all in fp32.
+// Reading W (25 MB at 6 x 4096 x 512) is the floor, 5 us; what is left is the
+// latency of one load, one silu phase and one reduction after the other, in a
+// single round of waves.  silu(t) of eight rows is formed once per workgroup; a
+// wave keeps it in registers (lane l: columns 8 l .. 8 l + 7 of each 512) and walks
+// over rows of W, kAdaRows of them loaded before the first is used; the eight sums
+// of a W row are reduced over the 64 lanes by halving first the sums a lane holds,
+// then the lanes.  8 frames, fp16: 23 us (34 us with a wait per loaded row), for
+// torch's conversions, GEMM and copies of the chunks 75 us and ten launches.
+constexpr int kAdaRows = 8;
+constexpr int kAdaWaves = 3072;  // three per SIMD
+
+struct AdaArgs {
+  const float* t;   // [R, K]
+  const void* w;    // [M, K]
+  const void* b;    // [M]
+  float* out;       // [M / C, R, C]
+  int32_t R, K, M, C;
+};
+
+template <typename T, int NC>
+__global__ __launch_bounds__(256) void adaln_kernel(AdaArgs p) {
+  const int wave = uniform_i32(blockIdx.x * 4 + threadIdx.x / 64);
+  const int lane = threadIdx.x % 64;
+  const int r0 = blockIdx.y * 8;
+  __shared__ __attribute__((aligned(16))) float silu[8][512 * NC];  // zero past R and K
+  {
+    constexpr int n = 512 * NC / 256;  // 256-column strips per row
+    float x[8 * n];
+#pragma unroll
+    for (int i = 0; i < 8 * n; ++i) {  // in-range loads, all before the first use
+      const int r = r0 + i / n, k = 256 * (i % n) + (int)threadIdx.x;
+      x[i] = p.t[(int64_t)(r < p.R ? r : 0) * p.K + (k < p.K ? k : 0)];
+    }
+#pragma unroll
+    for (int i = 0; i < 8 * n; ++i) {
+      const int r = i / n, k = 256 * (i % n) + (int)threadIdx.x;
+      const float v = r0 + r < p.R && k < p.K ? x[i] : 0.0f;
+      silu[r][k] = v / (1.0f + expf(-v));
+    }
+  }
+  __syncthreads();
+  float s[NC][8][8];
+#pragma unroll
+  for (int n = 0; n < NC; ++n)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) load8f(&silu[r][512 * n + 8 * lane], s[n][r]);
+  const int waves = gridDim.x * 4;
+  for (int m0 = wave * kAdaRows; m0 < p.M; m0 += waves * kAdaRows) {  // M % kAdaRows == 0
+    u32x4 raw[kAdaRows][NC];  // every load before the first use; zero past K
+#pragma unroll
+    for (int i = 0; i < kAdaRows; ++i)
+#pragma unroll
+      for (int n = 0; n < NC; ++n) {
+        const int k = 512 * n + 8 * lane;
+        raw[i][n] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const T*>(p.w) + (int64_t)(m0 + i) * p.K +
+                                                    (k < p.K ? k : 0));
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    float w[kAdaRows][NC][8];
+#pragma unroll
+    for (int i = 0; i < kAdaRows; ++i)
+#pragma unroll
+      for (int n = 0; n < NC; ++n)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t u = 512 * n + 8 * lane < p.K ? raw[i][n][e] : 0u;
+          w[i][n][2 * e] = to_f32(__builtin_bit_cast(T, (uint16_t)(u & 0xffffu)));
+          w[i][n][2 * e + 1] = to_f32(__builtin_bit_cast(T, (uint16_t)(u >> 16)));
+        }
+#pragma unroll
+    for (int i = 0; i < kAdaRows; ++i) {
+      float a[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        a[r] = 0.0f;
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) a[r] = __builtin_fmaf(s[n][r][e], w[i][n][e], a[r]);
+      }
+      // Lane bit 5 picks sums 0..3 or 4..7, bit 4 the pair, bit 3 the sum: lane l
+      // ends with sum (l / 8) over all lanes' columns.
+#pragma unroll
+      for (int h = 4, bit = 32; h >= 1; h /= 2, bit /= 2)
+#pragma unroll
+        for (int r = 0; r < h; ++r) {
+          const bool up = lane & bit;
+          const float mine = up ? a[r + h] : a[r], other = up ? a[r] : a[r + h];
+          a[r] = mine + __shfl_xor(other, bit);
+        }
+      const float sum = group_sum<8>(a[0]);
+      const int r = r0 + lane / 8;
+      const int m = m0 + i;
+      if (lane % 8 == 0 && r < p.R) {
+        const int j = m / p.C;
+        p.out[((int64_t)j * p.R + r) * p.C + (m - j * p.C)] = sum + to_f32(reinterpret_cast<const T*>(p.b)[m]);
+      }
+    }
+  }
+}
+
 }  // namespace
 
 bool rows_supported(int dtype, int C) { return dtype != 2 && C > 0 && C % 8 == 0 && C <= 8192; }
@@ -244,6 +348,25 @@ hipError_t launch_swiglu(const void* h, void* out, int dtype, int64_t rows, int 
   else
     hipLaunchKernelGGL((swiglu_kernel<bf16>), dim3(grid), dim3(256), 0, stream,
                        reinterpret_cast<const bf16*>(h), reinterpret_cast<bf16*>(out), rows, hidden);
+  return hipGetLastError();
+}
+
+bool adaln_supported(int dtype, int64_t K, int64_t C) {
+  return dtype != LCV_BSA_F32 && K > 0 && K % 8 == 0 && K <= 1024 && C > 0 && C % kAdaRows == 0;
+}
+
+hipError_t launch_adaln(const float* t, const void* w, const void* b, int dtype, int R, int K, int chunks, int C,
+                        float* out, hipStream_t stream) {
+  const AdaArgs p{t, w, b, out, R, K, chunks * C, C};
+  const int waves = std::min(p.M / kAdaRows, kAdaWaves);
+  const dim3 grid((unsigned)((waves + 3) / 4), (unsigned)((R + 7) / 8));
+  if (dtype == LCV_BSA_F16) {
+    if (K <= 512) hipLaunchKernelGGL((adaln_kernel<f16, 1>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((adaln_kernel<f16, 2>), grid, dim3(256), 0, stream, p);
+  } else {
+    if (K <= 512) hipLaunchKernelGGL((adaln_kernel<bf16, 1>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((adaln_kernel<bf16, 2>), grid, dim3(256), 0, stream, p);
+  }
   return hipGetLastError();
 }
 

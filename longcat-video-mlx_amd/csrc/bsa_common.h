@@ -249,6 +249,9 @@ hipError_t launch_rows(const void* x, const void* a, const float* gate, const fl
                        int tokens_per_frame, int frames, float eps, hipStream_t stream);
 hipError_t launch_swiglu(const void* h, void* out, int dtype, int64_t rows, int hidden,
                          hipStream_t stream);
+bool adaln_supported(int dtype, int64_t K, int64_t C);
+hipError_t launch_adaln(const float* t, const void* w, const void* b, int dtype, int R, int K, int chunks, int C,
+                        float* out, hipStream_t stream);
 hipError_t launch_head_norm(const void* x, const int64_t* xs, void* out, const int64_t* os,
                             const void* w, int dtype, int B, int N, int H, int D, float eps,
                             hipStream_t stream);

@@ -704,6 +704,25 @@ int lcv_bsa_block_swiglu(const void* h13, int dtype, int64_t rows, int64_t hidde
                        "lcv_bsa_block_swiglu");
 }
 
+int lcv_bsa_adaln(const float* t, const void* weight, const void* bias, int dtype, int64_t R, int64_t K,
+                  int64_t chunks, int64_t C, float* out, void* stream) {
+  if (!t || !weight || !bias || !out) return fail(LCV_BSA_ERR_INVALID_ARG, "null pointer");
+  if (dtype != LCV_BSA_F16 && dtype != LCV_BSA_BF16)
+    return fail(LCV_BSA_ERR_DTYPE, "adaln takes fp16 or bf16 weights (got dtype %d)", dtype);
+  if (R <= 0 || chunks <= 0 || R > kI32Max / 16 || chunks > 64 || C > kI32Max / 64)
+    return fail(LCV_BSA_ERR_SHAPE, "R=%lld, chunks=%lld or C=%lld out of range", (long long)R, (long long)chunks,
+                (long long)C);
+  if (!lcv::adaln_supported(dtype, K, C))
+    return fail(LCV_BSA_ERR_UNSUPPORTED, "adaln needs K %% 8 == 0, K <= 1024 and C %% 8 == 0 (K=%lld, C=%lld)",
+                (long long)K, (long long)C);
+  if ((uintptr_t)t % 16 || (uintptr_t)weight % 16)
+    return fail(LCV_BSA_ERR_LAYOUT, "t and weight must be 16-byte aligned");
+  if ((R + 7) / 8 > 65535) return fail(LCV_BSA_ERR_UNSUPPORTED, "R=%lld too large", (long long)R);
+  return launch_status(lcv::launch_adaln(t, weight, bias, dtype, (int)R, (int)K, (int)chunks, (int)C, out,
+                                         (hipStream_t)stream),
+                       "lcv_bsa_adaln");
+}
+
 int lcv_bsa_head_rms_norm(const void* x, int dtype, int64_t B, int64_t H, int64_t S, int64_t D,
                           lcv_bsa_strides xs, const void* weight, float eps, void* out,
                           lcv_bsa_strides os, void* stream) {

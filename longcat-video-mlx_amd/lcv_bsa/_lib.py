@@ -72,6 +72,8 @@ _SIGNATURES = {
                                    c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float,
                                    c_void_p, c_void_p, c_void_p]),
     "lcv_bsa_block_swiglu": (c_int, [c_void_p, c_int, c_int64, c_int64, c_void_p, c_void_p]),
+    "lcv_bsa_adaln": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, c_void_p,
+                              c_void_p]),
     "lcv_bsa_head_rms_norm": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int64, c_int64, Strides,
                                       c_void_p, c_float, c_void_p, Strides, c_void_p]),
     "lcv_bsa_text_attn": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64,

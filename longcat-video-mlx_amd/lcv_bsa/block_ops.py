@@ -6,7 +6,8 @@ the cross-attention pre-norm (longcat_video_dit.py:107-136; blocks.py:
 the cross-attention's per-head q / k norms (attention.py:325-326).  Each is
 one pass over HBM through ``liblcv_bsa.so``; each rounds like the
 reference's sequence of fp32 tensor operations followed by a cast.
-``text_attention`` is the cross-attention itself with the q norm inside
+``adaln_modulation`` gives the fp32 modulation of a timestep embedding
+(longcat_video_dit.py:80-138), ``text_attention`` is the cross-attention itself with the q norm inside
 (attention.py:318-352).
 """
 
@@ -20,7 +21,7 @@ import torch
 from . import _lib
 from .block_sparse_attention import _dtype_code, _require_device, _stream, _strides
 
-__all__ = ["residual_norm", "swiglu", "head_rms_norm", "text_attention", "plain_tensors"]
+__all__ = ["residual_norm", "swiglu", "head_rms_norm", "adaln_modulation", "text_attention", "plain_tensors"]
 
 
 def plain_tensors(*ts: Optional[torch.Tensor]) -> bool:
@@ -124,6 +125,22 @@ def head_rms_norm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float = 
         x.data_ptr(), _dtype_code(x), B, H, S, D, _strides(x), _ptr(weight), float(eps),
         out.data_ptr(), _strides(out), _stream(x))
     _lib.check(st, "head_rms_norm")
+    return out
+
+
+def adaln_modulation(t: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, chunks: int) -> torch.Tensor:
+    """``silu(t) @ weight^T + bias`` in fp32 for ``t`` ``[B, T, K]`` fp32 and a
+    half-precision ``weight`` ``[chunks * C, K]``: ``[chunks, B, T, C]``."""
+    _require_device(t, weight, bias)
+    B, T, K = t.shape
+    C = weight.shape[0] // chunks
+    if t.dtype != torch.float32 or bias.dtype != weight.dtype:
+        raise ValueError(f"t must be fp32 and bias of weight's dtype, got {t.dtype}, {bias.dtype}, {weight.dtype}")
+    t, weight, bias = t.contiguous(), _rows(weight, "weight", (chunks * C, K)), _rows(bias, "bias", (chunks * C,))
+    out = torch.empty((chunks, B, T, C), dtype=torch.float32, device=t.device)
+    st = _lib.load().lcv_bsa_adaln(t.data_ptr(), weight.data_ptr(), bias.data_ptr(), _dtype_code(weight), B * T, K,
+                                   chunks, C, out.data_ptr(), _stream(t))
+    _lib.check(st, "adaln_modulation")
     return out
 
 

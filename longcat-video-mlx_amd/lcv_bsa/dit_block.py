@@ -24,7 +24,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .attention import BSAAttention, dense_attention, validate_backend
-from .block_ops import head_rms_norm, plain_tensors, residual_norm, swiglu, text_attention
+from .block_ops import adaln_modulation, head_rms_norm, plain_tensors, residual_norm, swiglu, text_attention
 from .block_sparse_attention import bsa_attention
 from .prepare import prepare_qk, prepare_qkv
 from .rope_3d import rope_3d
@@ -387,6 +387,21 @@ class LongCatSingleStreamBlock(nn.Module):
         # HIP row passes (same fp32 arithmetic as the unfused path below).
         self.fused = True
 
+    def _modulation(self, t, fused):
+        """The six fp32 chunks [B, T, 1, C] of ``silu(t) W^T + b``
+        (longcat_video_dit.py:80-138); on the fused path one kernel."""
+        lin = self.adaLN_modulation[1]
+        w, b = lin.weight, lin.bias
+        if (fused and t.dim() == 3 and t.is_cuda and w.device == b.device == t.device
+                and w.dtype == b.dtype and w.dtype in (torch.float16, torch.bfloat16)
+                and w.data_ptr() % 16 == 0 and w.is_contiguous() and w.shape[0] == 6 * self.hidden_size
+                and t.shape[-1] == w.shape[1] <= 1024 and w.shape[1] % 8 == 0
+                and not torch.is_autocast_enabled("cuda")):
+            tf = t.float()
+            if tf.data_ptr() % 16 == 0:
+                return adaln_modulation(tf, w, b, 6).unsqueeze(3).unbind(0)
+        return F.linear(F.silu(t.float()), w.float(), b.float())[:, :, None, :].chunk(6, dim=-1)
+
     def _self_attn(self, x_m, latent_shape, num_cond_latents, return_kv, kv_cache):
         if kv_cache is not None:
             return self.attn.forward_with_kv_cache(x_m, latent_shape, num_cond_latents, kv_cache), kv_cache
@@ -397,7 +412,7 @@ class LongCatSingleStreamBlock(nn.Module):
     def _forward_fused(self, x, y, t, y_seqlen, latent_shape, num_cond_latents, return_kv, kv_cache,
                        skip_crs_attn, ada):
         T = int(latent_shape[0])
-        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = ada.chunk(6, dim=-1)
+        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = ada
         _, x_m = residual_norm(x, frames=T, shift=shift_msa, scale=scale_msa, eps=self.mod_norm_attn.eps)
         x_s, new_kv = self._self_attn(x_m, latent_shape, num_cond_latents, return_kv, kv_cache)
         pre = self.pre_crs_attn_norm
@@ -421,13 +436,12 @@ class LongCatSingleStreamBlock(nn.Module):
         dtype = x.dtype
         B, N, C = x.shape
         T = int(latent_shape[0])
-        lin = self.adaLN_modulation[1]
-        ada = F.linear(F.silu(t.float()), lin.weight.float(), lin.bias.float())[:, :, None, :]
-        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = ada.chunk(6, dim=-1)
-
-        if self.fused and x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and C % 8 == 0:
+        fused = self.fused and x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and C % 8 == 0
+        ada = self._modulation(t, fused)
+        if fused:
             return self._forward_fused(x, y, t, y_seqlen, latent_shape, num_cond_latents, return_kv, kv_cache,
                                        skip_crs_attn, ada)
+        shift_msa, scale_msa, gate_msa, shift_mlp, scale_mlp, gate_mlp = ada
         x_m = modulate_fp32(self.mod_norm_attn, x.view(B, T, -1, C), shift_msa, scale_msa).view(B, N, C)
         x_s, new_kv = self._self_attn(x_m, latent_shape, num_cond_latents, return_kv, kv_cache)
         x = (x.float() + (gate_msa * x_s.view(B, T, -1, C).float()).view(B, N, C)).to(dtype)
