@@ -62,9 +62,27 @@ __device__ __forceinline__ void load8f(const float* p, float* v) {
   v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
 }
 
+template <typename T>
+__device__ __forceinline__ void widen8(const u32x4& raw, float* v) {
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const uint32_t w = raw[m];
+    v[2 * m] = to_f32(__builtin_bit_cast(T, (uint16_t)(w & 0xffffu)));
+    v[2 * m + 1] = to_f32(__builtin_bit_cast(T, (uint16_t)(w >> 16)));
+  }
+}
+
 // One wave per row; lane l holds the 8-element chunks l, l + 64, ... of the
-// row (NMAX chunks at most, so C <= 512 * NMAX).
-template <typename T, int NMAX>
+// row (NMAX chunks at most, so C <= 512 * NMAX).  HBM bound: all of a row's x and a
+// are loaded before the first use, and nothing in the kernel branches per lane
+// (a chunk past the row re-reads the lane's first one and counts for nothing), so
+// that no load waits for another.  28,800 x 4096, fp16, before (a wait per chunk and
+// tensor) and now: gated residual + norm 192 -> 179 us (5.3 TB/s), residual +
+// modulation 196 -> 178, modulation alone 115 -> 104, gated residual alone 131 -> 126;
+// at C = 8192 451 -> 345, 440 -> 352, 265 -> 232 and 306 -> 251 us.
+enum RowMode { kNoAdd = 0, kAdd = 1, kGatedAdd = 2 };
+
+template <typename T, int NMAX, int MODE>
 __global__ __launch_bounds__(256) void rows_kernel(RowArgs p) {
   const int wave = uniform_i32(threadIdx.x / 64);
   const int lane = threadIdx.x % 64;
@@ -75,26 +93,42 @@ __global__ __launch_bounds__(256) void rows_kernel(RowArgs p) {
   const int64_t frame = ((int64_t)b * p.frames + t) * p.C;
   const int64_t base = (int64_t)row * p.C;
   const int nch = p.C / 8;
+  const int first = lane < nch ? lane : 0;
+  auto chunk = [&](int i) { return lane + 64 * i < nch ? lane + 64 * i : first; };
+  auto live = [&](int i) { return lane + 64 * i < nch; };
 
+  u32x4 xr[NMAX], ar[NMAX];
+#pragma unroll
+  for (int i = 0; i < NMAX; ++i)
+    xr[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const T*>(p.x) + base + 8 * chunk(i));
+  if constexpr (MODE != kNoAdd) {
+#pragma unroll
+    for (int i = 0; i < NMAX; ++i)
+      ar[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const T*>(p.a) + base + 8 * chunk(i));
+  }
   float r[NMAX][8];
 #pragma unroll
   for (int i = 0; i < NMAX; ++i) {
-    const int c = lane + 64 * i;
-    if (c >= nch) break;
-    load8(reinterpret_cast<const T*>(p.x) + base + 8 * c, r[i]);
-    if (p.a) {
+    widen8<T>(xr[i], r[i]);
+    if constexpr (MODE != kNoAdd) {
       float av[8];
-      load8(reinterpret_cast<const T*>(p.a) + base + 8 * c, av);
-      if (p.gate) {
+      widen8<T>(ar[i], av);
+      if constexpr (MODE == kGatedAdd) {
         float g[8];
-        load8f(p.gate + frame + 8 * c, g);
+        load8f(p.gate + frame + 8 * chunk(i), g);
 #pragma unroll
         for (int e = 0; e < 8; ++e) r[i][e] = to_f32(round_from_f32<T>(r[i][e] + g[e] * av[e]));
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e) r[i][e] = to_f32(round_from_f32<T>(r[i][e] + av[e]));
       }
-      if (p.x_out) store8(reinterpret_cast<T*>(p.x_out) + base + 8 * c, r[i]);
+    }
+  }
+  if constexpr (MODE != kNoAdd) {
+    if (p.x_out) {
+#pragma unroll
+      for (int i = 0; i < NMAX; ++i)
+        if (live(i)) store8(reinterpret_cast<T*>(p.x_out) + base + 8 * chunk(i), r[i]);
     }
   }
   if (!p.n_out) return;
@@ -102,73 +136,109 @@ __global__ __launch_bounds__(256) void rows_kernel(RowArgs p) {
   // LayerNorm in fp32: mean, then the mean of squared deviations.
   float s = 0.0f;
 #pragma unroll
-  for (int i = 0; i < NMAX; ++i) {
-    if (lane + 64 * i >= nch) break;
+  for (int i = 0; i < NMAX; ++i)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) s += r[i][e];
-  }
+    for (int e = 0; e < 8; ++e) s += live(i) ? r[i][e] : 0.0f;
   const float mean = wave_sum(s) / (float)p.C;
   float q = 0.0f;
 #pragma unroll
-  for (int i = 0; i < NMAX; ++i) {
-    if (lane + 64 * i >= nch) break;
+  for (int i = 0; i < NMAX; ++i)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const float d = r[i][e] - mean;
+      const float d = live(i) ? r[i][e] - mean : 0.0f;
       q += d * d;
     }
-  }
   const float rstd = rsqrtf(wave_sum(q) / (float)p.C + p.eps);
 #pragma unroll
-  for (int i = 0; i < NMAX; ++i) {
-    const int c = lane + 64 * i;
-    if (c >= nch) break;
-    float y[8];
+  for (int i = 0; i < NMAX; ++i)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = (r[i][e] - mean) * rstd;
-    if (p.ln_w) {
+    for (int e = 0; e < 8; ++e) r[i][e] = (r[i][e] - mean) * rstd;
+  if (p.ln_w) {
+#pragma unroll
+    for (int i = 0; i < NMAX; ++i) {
       float w[8], bb[8];
-      load8(reinterpret_cast<const T*>(p.ln_w) + 8 * c, w);
-      load8(reinterpret_cast<const T*>(p.ln_b) + 8 * c, bb);
+      load8(reinterpret_cast<const T*>(p.ln_w) + 8 * chunk(i), w);
+      load8(reinterpret_cast<const T*>(p.ln_b) + 8 * chunk(i), bb);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = y[e] * w[e] + bb[e];
+      for (int e = 0; e < 8; ++e) r[i][e] = r[i][e] * w[e] + bb[e];
     }
-    if (p.scale) {
-      float sc[8], sh[8];
-      load8f(p.scale + frame + 8 * c, sc);
-      load8f(p.shift + frame + 8 * c, sh);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = y[e] * (sc[e] + 1.0f) + sh[e];
-    }
-    store8(reinterpret_cast<T*>(p.n_out) + base + 8 * c, y);
   }
+  if (p.scale) {
+#pragma unroll
+    for (int i = 0; i < NMAX; ++i) {
+      float sc[8], sh[8];
+      load8f(p.scale + frame + 8 * chunk(i), sc);
+      load8f(p.shift + frame + 8 * chunk(i), sh);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) r[i][e] = r[i][e] * (sc[e] + 1.0f) + sh[e];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NMAX; ++i)
+    if (live(i)) store8(reinterpret_cast<T*>(p.n_out) + base + 8 * chunk(i), r[i]);
+}
+
+template <typename T, int NMAX, int MODE>
+hipError_t launch_rows_m(const RowArgs& a, hipStream_t stream) {
+  const int grid = (a.rows + kRowWaves - 1) / kRowWaves;
+  hipLaunchKernelGGL((rows_kernel<T, NMAX, MODE>), dim3(grid), dim3(64 * kRowWaves), 0, stream, a);
+  return hipGetLastError();
 }
 
 template <typename T, int NMAX>
 hipError_t launch_rows_t(const RowArgs& a, hipStream_t stream) {
-  const int grid = (a.rows + kRowWaves - 1) / kRowWaves;
-  hipLaunchKernelGGL((rows_kernel<T, NMAX>), dim3(grid), dim3(64 * kRowWaves), 0, stream, a);
-  return hipGetLastError();
+  if (!a.a) return launch_rows_m<T, NMAX, kNoAdd>(a, stream);
+  return a.gate ? launch_rows_m<T, NMAX, kGatedAdd>(a, stream) : launch_rows_m<T, NMAX, kAdd>(a, stream);
 }
 
 // silu(a) * b, each rounded to the dtype (torch's silu computes x / (1 +
 // exp(-x)) in fp32; the product of two dtype values is exact in fp32).
+// Inside |x| < 80 the division runs as a reciprocal, a product and one residual
+// correction, the quotient that IEEE division gives (checked for every fp16 and
+// bf16 x), without its scaling of extreme operands; waves with larger x divide.
+// With a 64-bit division per thread for its row the kernel was bound by the VALU:
+// 28,800 x 11,008, fp16, 384 -> 343 us (5.5 TB/s, the rate of a copy).
+__device__ __forceinline__ float silu_near(float x) {
+  const float d = 1.0f + expf(-x);
+  const float rc = __builtin_amdgcn_rcpf(d);
+  const float y = x * rc;
+  return __builtin_fmaf(-__builtin_fmaf(d, y, -x), rc, y);  // this order of signs keeps -0
+}
+
+constexpr int kGatePer = 2;  // 8-element chunks per thread
+
 template <typename T>
-__global__ __launch_bounds__(256) void swiglu_kernel(const T* h, T* out, int64_t rows, int32_t hidden) {
-  const int64_t n8 = rows * (hidden / 8);
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n8) return;
-  const int64_t row = i / (hidden / 8);
-  const int c = (int)(i - row * (hidden / 8));
-  float a[8], bv[8], y[8];
-  load8(h + row * 2 * hidden + 8 * c, a);
-  load8(h + row * 2 * hidden + hidden + 8 * c, bv);
+__global__ __launch_bounds__(256) void swiglu_kernel(const T* h, T* out, uint32_t n8, FastDiv per_row) {
+  u32x4 ar[kGatePer], br[kGatePer];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float s = to_f32(round_from_f32<T>(a[e] / (1.0f + expf(-a[e]))));
-    y[e] = s * bv[e];
+  for (int u = 0; u < kGatePer; ++u) {
+    const uint32_t i = (blockIdx.x * kGatePer + u) * 256u + threadIdx.x;
+    const uint32_t j = i < n8 ? i : n8 - 1;
+    const uint32_t row = fast_div(j, per_row);
+    const T* src = h + 8 * ((int64_t)row * per_row.d + j);
+    ar[u] = *reinterpret_cast<const u32x4*>(src);
+    br[u] = *reinterpret_cast<const u32x4*>(src + 8 * (int64_t)per_row.d);
   }
-  store8(out + row * hidden + 8 * c, y);
+#pragma unroll
+  for (int u = 0; u < kGatePer; ++u) {
+    const uint32_t i = (blockIdx.x * kGatePer + u) * 256u + threadIdx.x;
+    float a[8], bv[8], y[8];
+    widen8<T>(ar[u], a);
+    widen8<T>(br[u], bv);
+    float m = 0.0f;  // a NaN is no maximum: silu_near keeps it
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(a[e]));
+    if (__ballot(!(m < 80.0f))) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = a[e] / (1.0f + expf(-a[e]));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = silu_near(a[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = to_f32(round_from_f32<T>(y[e])) * bv[e];
+    if (i < n8) store8(out + 8 * (int64_t)i, y);
+  }
 }
 
 // RMSNorm_FP32 of rows of D elements: (b, n, h) -> out[b, h, n, :] (any
@@ -330,10 +400,12 @@ hipError_t launch_rows(const void* x, const void* a, const float* gate, const fl
   const int nmax = (C / 8 + 63) / 64;
   if (dtype == 0) {
     if (nmax <= 2) return launch_rows_t<f16, 2>(p, stream);
+    if (nmax <= 4) return launch_rows_t<f16, 4>(p, stream);
     if (nmax <= 8) return launch_rows_t<f16, 8>(p, stream);
     return launch_rows_t<f16, 16>(p, stream);
   }
   if (nmax <= 2) return launch_rows_t<bf16, 2>(p, stream);
+  if (nmax <= 4) return launch_rows_t<bf16, 4>(p, stream);
   if (nmax <= 8) return launch_rows_t<bf16, 8>(p, stream);
   return launch_rows_t<bf16, 16>(p, stream);
 }
@@ -341,13 +413,15 @@ hipError_t launch_rows(const void* x, const void* a, const float* gate, const fl
 hipError_t launch_swiglu(const void* h, void* out, int dtype, int64_t rows, int hidden,
                          hipStream_t stream) {
   const int64_t n8 = rows * (hidden / 8);
-  const int grid = (int)((n8 + 255) / 256);
+  if (n8 > 0xFFFFFFFFll - 256 * kGatePer) return hipErrorInvalidValue;
+  const int grid = (int)((n8 + 256 * kGatePer - 1) / (256 * kGatePer));
+  const FastDiv per_row = make_fastdiv((uint32_t)(hidden / 8));
   if (dtype == 0)
     hipLaunchKernelGGL((swiglu_kernel<f16>), dim3(grid), dim3(256), 0, stream,
-                       reinterpret_cast<const f16*>(h), reinterpret_cast<f16*>(out), rows, hidden);
+                       reinterpret_cast<const f16*>(h), reinterpret_cast<f16*>(out), (uint32_t)n8, per_row);
   else
     hipLaunchKernelGGL((swiglu_kernel<bf16>), dim3(grid), dim3(256), 0, stream,
-                       reinterpret_cast<const bf16*>(h), reinterpret_cast<bf16*>(out), rows, hidden);
+                       reinterpret_cast<const bf16*>(h), reinterpret_cast<bf16*>(out), (uint32_t)n8, per_row);
   return hipGetLastError();
 }
 
