@@ -49,6 +49,22 @@ __device__ __forceinline__ T round_from_f32(float v) {
   return from_f32<T>(v);
 }
 
+// Two fp32 results rounded to T as round_from_f32 does, packed (the first in the
+// low half): one v_cvt_pk_bf16_f32 for bf16.
+template <typename T>
+__device__ __forceinline__ uint32_t round_pair(float a, float b);
+template <>
+__device__ __forceinline__ uint32_t round_pair<f16>(float a, float b) {
+  return bits16(round_from_f32<f16>(a)) | (bits16(round_from_f32<f16>(b)) << 16);
+}
+template <>
+__device__ __forceinline__ uint32_t round_pair<bf16>(float a, float b) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  const f2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2));
+}
+
 // RMSNorm_FP32's output: round(x * rs) to T, times the weight, rounded to T
 // (an exact product of two T values rounded once, so fp16 uses the packed
 // fp16 multiply).
@@ -74,9 +90,11 @@ __device__ __forceinline__ void norm_scale<bf16>(const float* x, float rs, u32x4
   for (int m = 0; m < 4; ++m) {
     const uint32_t wm = wr[m];
     const float w0 = __builtin_bit_cast(float, wm << 16), w1 = __builtin_bit_cast(float, wm & 0xffff0000u);
-    y[2 * m] = to_f32(round_from_f32<bf16>(mul1(to_f32(round_from_f32<bf16>(mul1(x[2 * m], rs, nz))), w0, nz)));
-    y[2 * m + 1] =
-        to_f32(round_from_f32<bf16>(mul1(to_f32(round_from_f32<bf16>(mul1(x[2 * m + 1], rs, nz))), w1, nz)));
+    const uint32_t n = round_pair<bf16>(mul1(x[2 * m], rs, nz), mul1(x[2 * m + 1], rs, nz));
+    const uint32_t o = round_pair<bf16>(mul1(__builtin_bit_cast(float, n << 16), w0, nz),
+                                        mul1(__builtin_bit_cast(float, n & 0xffff0000u), w1, nz));
+    y[2 * m] = __builtin_bit_cast(float, o << 16);
+    y[2 * m + 1] = __builtin_bit_cast(float, o & 0xffff0000u);
   }
 }
 

@@ -86,25 +86,39 @@ __device__ __forceinline__ int lds_slot(const PrepArgs& a, int i) {
 }
 
 // What a lane needs to turn rows: per pair p (dims 8c + 2p, +1) its axis and its
-// column's offset in that axis' LDS row (in floats).
+// column's byte offset in that axis' LDS row.
 template <int D>
 struct RopeLane {
-  int axis[4], col2[4];
-  int ht2, hh2, hw2;  // floats per LDS row of each axis
-  int reg_h, reg_w;
-  uint32_t plane;
+  int axis[4], col[4];
   __device__ RopeLane(const PrepArgs& a, int c) {
-    ht2 = a.dt, hh2 = a.dh, hw2 = D - a.dt - a.dh;
-    reg_h = a.rT * ht2, reg_w = reg_h + a.rH * hh2;
 #pragma unroll
     for (int pp = 0; pp < 4; ++pp) {
       const int d = 8 * c + 2 * pp;
       axis[pp] = d < a.dt ? 0 : (d < a.dt + a.dh ? 1 : 2);
-      col2[pp] = axis[pp] == 0 ? d : (axis[pp] == 1 ? d - a.dt : d - a.dt - a.dh);
+      col[pp] = 4 * (axis[pp] == 0 ? d : (axis[pp] == 1 ? d - a.dt : d - a.dt - a.dh));
     }
-    plane = (uint32_t)(a.rH * a.rW);
   }
 };
+
+// Where the LDS rows of grid position `tok` start, per axis, in (cos, sin) pairs
+// (below kMaxRopeTable / 2).  One lane per row of a block computes it, for the D / 8
+// lanes that turn the row (each of them for itself, and with unpacked bf16
+// rounding, a step was 215 to 269 instructions, now 156 to 164, and the VALU the
+// bound beside HBM): filling a cache of 28,800 tokens x 32 heads x 128 263 -> 230 us
+// (5.1 TB/s); D = 64, 20,480 x 16: q and k 40.3 -> 35.0 us, around a cache 79 -> 67.
+struct RopePos {
+  uint16_t slot[4];
+};
+__device__ __forceinline__ RopePos rope_pos(const PrepArgs& a, uint32_t tok) {
+  const uint32_t ht = (uint32_t)a.dt / 2, hh = (uint32_t)a.dh / 2, hw = (uint32_t)(a.D - a.dt - a.dh) / 2;
+  const uint32_t pt = small_div(tok, a.rcp_plane);
+  const uint32_t prem = tok - __umul24(pt, (uint32_t)(a.rH * a.rW));
+  const uint32_t ph = small_div(prem, a.rcp_w);
+  const uint32_t pw = prem - __umul24(ph, (uint32_t)a.rW);
+  const uint32_t reg_h = (uint32_t)a.rT * ht, reg_w = reg_h + (uint32_t)a.rH * hh;
+  return RopePos{{(uint16_t)__umul24(pt, ht), (uint16_t)(reg_h + __umul24(ph, hh)),
+                  (uint16_t)(reg_w + __umul24(pw, hw)), 0}};
+}
 
 template <typename T>
 __device__ __forceinline__ u32x4 load_weight(const void* w, int c) {
@@ -135,31 +149,25 @@ __device__ __forceinline__ void norm_row(const float (&x)[8], const u32x4& wr, f
   norm_scale<T>(x, rs, wr, nz, y);
 }
 
-// RoPE of y at grid position `tok`; the rounded row is packed and added to acc.
+// RoPE of y at the position whose slots are `pos`; the rounded row is packed and
+// added to acc.
 template <typename T, int D>
-__device__ __forceinline__ u32x4 rope_row(const PrepArgs& a, const RopeLane<D>& L, const float* tab, uint32_t tok,
-                                          const float (&y)[8], float (&acc)[8]) {
-  const uint32_t pt = small_div(tok, a.rcp_plane);
-  const uint32_t prem = tok - __umul24(pt, L.plane);
-  const uint32_t ph = small_div(prem, a.rcp_w);
-  const uint32_t pw = prem - __umul24(ph, (uint32_t)a.rW);
-  const int at = (int)__umul24(pt, (uint32_t)L.ht2);
-  const int ah = L.reg_h + (int)__umul24(ph, (uint32_t)L.hh2);
-  const int aw = L.reg_w + (int)__umul24(pw, (uint32_t)L.hw2);
+__device__ __forceinline__ u32x4 rope_row(const PrepArgs& a, const RopeLane<D>& L, const float* tab,
+                                          const RopePos& pos, const float (&y)[8], float (&acc)[8]) {
   const float nz = a.neg_zero, one = a.one;
   uint32_t packed[4];
 #pragma unroll
   for (int pp = 0; pp < 4; ++pp) {
-    const int slot = (L.axis[pp] == 0 ? at : (L.axis[pp] == 1 ? ah : aw)) + L.col2[pp];
-    const float2 f = *reinterpret_cast<const float2*>(tab + slot);
+    const float2 f = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(tab) +
+                                                      (8 * (int)pos.slot[L.axis[pp]] + L.col[pp]));
     const float cs = f.x, sn = f.y;
     const float u = y[2 * pp], v = y[2 * pp + 1];
     // x*cos + rotate_half(x)*sin, rounded per product and sum.
-    const T o0 = round_from_f32<T>(mul1(u, cs, nz) - mul1(v, sn, nz));
-    const T o1 = round_from_f32<T>(mul1(v, cs, nz) + mul1(u, sn, nz));
+    packed[pp] = round_pair<T>(mul1(u, cs, nz) - mul1(v, sn, nz), mul1(v, cs, nz) + mul1(u, sn, nz));
+    const T o0 = __builtin_bit_cast(T, (uint16_t)(packed[pp] & 0xffffu));
+    const T o1 = __builtin_bit_cast(T, (uint16_t)(packed[pp] >> 16));
     acc[2 * pp] = __builtin_fmaf(to_f32(o0), one, acc[2 * pp]);
     acc[2 * pp + 1] = __builtin_fmaf(to_f32(o1), one, acc[2 * pp + 1]);
-    packed[pp] = bits16(o0) | (bits16(o1) << 16);
   }
   return u32x4{packed[0], packed[1], packed[2], packed[3]};
 }
@@ -182,13 +190,32 @@ __device__ __forceinline__ void store_mean(float (&acc)[8], float* mean, int lan
   }
 }
 
+// Row loads in flight per lane and waves per SIMD at least.  D = 128: 2 and 6 (4 and 4
+// gave 380 against 380 us for q, k of 57,600 tokens x 32 heads, 198 / 194 us at
+// 28,800, 398 / 387 us around a cache); D = 64: 4 and 4 (34.5 against 35.8 us at
+// 20,480 x 16, 67 / 73 us around a cache).
+template <int D>
+struct PrepTune {
+  static constexpr int kBatch = D == 128 ? 2 : 4, kWaves = D == 128 ? 6 : 4;
+};
+
+// Lane l's slots to row l of this wave's table.  LDS operations of one wave complete
+// in order; the fences keep the compiler from moving reads across.
+__device__ __forceinline__ void set_pos(RopePos* pos, int lane, const RopePos& v) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  pos[lane] = v;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 template <typename T, int D>
-__global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PrepTune<D>::kWaves))) void prep_kernel(PrepArgs a) {
   constexpr int LPR = D / 8;       // lanes per row (8 elements per lane)
   constexpr int RPS = 64 / LPR;    // rows per step
+  constexpr int kPrepBatch = PrepTune<D>::kBatch;
   extern __shared__ float tab[];  // table_len floats (dynamic)
   __shared__ int64_t row_in[2][64], row_out[2][64];  // element offset of each block row
-  __shared__ int32_t row_tok[64];                    // token offset of each block row
+  __shared__ RopePos pos[kPrepWaves][64];            // of a wave's block rows
 
   // The workgroup is persistent: the table and the row offsets are staged
   // once and its waves then walk the (block, tensor, b, h) items with a
@@ -196,7 +223,6 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
   for (int i = threadIdx.x; i < a.table_len; i += 256) tab[lds_slot(a, i)] = a.table[i];
   if (threadIdx.x < 64) {
     const int32_t t = voxel_row_offset(a.g, threadIdx.x);
-    row_tok[threadIdx.x] = t;
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       row_in[k][threadIdx.x] = (int64_t)t * a.in[k].ss;
@@ -209,6 +235,7 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
   const int lane = threadIdx.x % 64;
   const int c = lane % LPR;  // this lane's 8 dims: 8c .. 8c+7
   const RopeLane<D> L(a, c);
+  const uint32_t lane_tok = (uint32_t)voxel_row_offset(a.g, lane);
   const int stride = gridDim.x * kPrepWaves;
 
   for (int item = blockIdx.x * kPrepWaves + wave; item < a.total_items; item += stride) {
@@ -229,20 +256,29 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
     T* dst = reinterpret_cast<T*>(const_cast<void*>(xo.ptr)) + (int64_t)b * xo.sb + (int64_t)h * xo.sh +
              (int64_t)tok0 * xo.ss + 8 * c;
     const u32x4 wr = load_weight<T>(a.weight[tensor], c);
+    set_pos(pos[wave], lane, rope_pos(a, (uint32_t)tok0 + lane_tok));
 
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
-#pragma unroll 2
-    for (int st = 0; st < 64 / RPS; ++st) {
-      const int row = st * RPS + lane / LPR;
+#pragma unroll 1
+    for (int s0 = 0; s0 < 64 / RPS; s0 += kPrepBatch) {
       // q / k are streamed once: non-temporal loads and stores.
-      const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + row_in[tensor][row]));
-      float x[8], y[8];
-      widen8<T>(raw, x);
-      norm_row<T, D>(x, wr, a.eps, a.neg_zero, y);
-      const u32x4 packed = rope_row<T, D>(a, L, tab, (uint32_t)(tok0 + row_tok[row]), y, acc);
-      __builtin_nontemporal_store(packed, reinterpret_cast<u32x4*>(dst + row_out[tensor][row]));
+      u32x4 raw[kPrepBatch];
+#pragma unroll
+      for (int u = 0; u < kPrepBatch; ++u)
+        raw[u] = __builtin_nontemporal_load(
+            reinterpret_cast<const u32x4*>(src + row_in[tensor][(s0 + u) * RPS + lane / LPR]));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < kPrepBatch; ++u) {
+        const int row = (s0 + u) * RPS + lane / LPR;
+        float x[8], y[8];
+        widen8<T>(raw[u], x);
+        norm_row<T, D>(x, wr, a.eps, a.neg_zero, y);
+        const u32x4 packed = rope_row<T, D>(a, L, tab, pos[wave][row], y, acc);
+        __builtin_nontemporal_store(packed, reinterpret_cast<u32x4*>(dst + row_out[tensor][row]));
+      }
     }
     store_mean<D>(acc, a.mean[tensor] + ((int64_t)bh * a.nb + n) * D, lane);
   }
@@ -255,15 +291,17 @@ __global__ __launch_bounds__(256) void prep_kernel(PrepArgs a) {
 // run k-block (v-block) by k-block; the last nb of the nk k-blocks go with the
 // q-blocks, so that the rows of a token that q, k and v share are read together.
 // HBM bound, as prep_kernel.  Measured at 32 heads of 128, bf16, 3,600 tokens a
-// frame: 8 frames after 4 cached ones 1.89 GB in 0.40 ms, 4.7 TB/s (the torch
+// frame: 8 frames after 4 cached ones 1.89 GB in 0.39 ms, 4.9 TB/s (the torch
 // norms, concatenations and RoPE it replaces: 7.3 ms); filling a cache of 4
-// frames 0.59 GB in 0.15 ms (2.3 ms).
+// frames 0.59 GB in 0.14 ms (2.3 ms).
 template <typename T, int D>
-__global__ __launch_bounds__(256) void prep_cached_kernel(CachedArgs ca) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PrepTune<D>::kWaves))) void prep_cached_kernel(CachedArgs ca) {
   constexpr int LPR = D / 8;
   constexpr int RPS = 64 / LPR;
+  constexpr int kPrepBatch = PrepTune<D>::kBatch;
   extern __shared__ float tab[];
-  __shared__ int32_t row_tok[2][64];  // token offset of each block row: q's geometry, k's
+  __shared__ int32_t row_tok[2][64];       // token offset of each block row: q's geometry, k's
+  __shared__ RopePos pos[kPrepWaves][64];  // of a wave's block rows
   const PrepArgs& a = ca.p;
   for (int i = threadIdx.x; i < a.table_len; i += 256) tab[lds_slot(a, i)] = a.table[i];
   if (threadIdx.x < 64) {
@@ -319,30 +357,40 @@ __global__ __launch_bounds__(256) void prep_cached_kernel(CachedArgs ca) {
                                           (int64_t)b * ca.k_norm.sb + (int64_t)h * ca.k_norm.sh + 8 * c
                                     : nullptr;
     const u32x4 wr = load_weight<T>(a.weight[tensor], c);
+    set_pos(pos[wave], lane, rope_pos(a, (uint32_t)(tok0 + rows[lane] + (tensor ? 0 : ca.cached))));
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
-#pragma unroll 2
-    for (int st = 0; st < 64 / RPS; ++st) {
-      const int32_t t = tok0 + rows[st * RPS + lane / LPR];
-      const bool is_new = t >= first_new;
-      const T* from = is_new ? src + (int64_t)(t - first_new) * xi.ss : old + (int64_t)t * xc.ss;
-      const u32x4 raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(from));
-      float x[8], y[8];
-      widen8<T>(raw, x);
-      norm_row<T, D>(x, wr, a.eps, a.neg_zero, y);
-      if (kn && is_new) {
-        uint32_t w[4];
+#pragma unroll 1
+    for (int s0 = 0; s0 < 64 / RPS; s0 += kPrepBatch) {
+      u32x4 raw[kPrepBatch];
 #pragma unroll
-        for (int m = 0; m < 4; ++m)  // exact: y holds T values
-          w[m] = bits16(from_f32<T>(y[2 * m])) | (bits16(from_f32<T>(y[2 * m + 1])) << 16);
-        *reinterpret_cast<u32x4*>(kn + (int64_t)(t - first_new) * ca.k_norm.ss) = u32x4{w[0], w[1], w[2], w[3]};
+      for (int u = 0; u < kPrepBatch; ++u) {
+        const int32_t t = tok0 + rows[(s0 + u) * RPS + lane / LPR];
+        const T* from = t >= first_new ? src + (int64_t)(t - first_new) * xi.ss : old + (int64_t)t * xc.ss;
+        raw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(from));
       }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = is_new ? y[e] : x[e];
-      const uint32_t pos = (uint32_t)(tensor ? t : t + ca.cached);
-      const u32x4 packed = rope_row<T, D>(a, L, tab, pos, y, acc);
-      __builtin_nontemporal_store(packed, reinterpret_cast<u32x4*>(dst + (int64_t)t * xo.ss));
+      for (int u = 0; u < kPrepBatch; ++u) {
+        const int row = (s0 + u) * RPS + lane / LPR;
+        const int32_t t = tok0 + rows[row];
+        const bool is_new = t >= first_new;
+        float x[8], y[8];
+        widen8<T>(raw[u], x);
+        norm_row<T, D>(x, wr, a.eps, a.neg_zero, y);
+        if (kn && is_new) {
+          uint32_t w[4];
+#pragma unroll
+          for (int m = 0; m < 4; ++m)  // exact: y holds T values
+            w[m] = bits16(from_f32<T>(y[2 * m])) | (bits16(from_f32<T>(y[2 * m + 1])) << 16);
+          *reinterpret_cast<u32x4*>(kn + (int64_t)(t - first_new) * ca.k_norm.ss) = u32x4{w[0], w[1], w[2], w[3]};
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = is_new ? y[e] : x[e];
+        const u32x4 packed = rope_row<T, D>(a, L, tab, pos[wave][row], y, acc);
+        __builtin_nontemporal_store(packed, reinterpret_cast<u32x4*>(dst + (int64_t)t * xo.ss));
+      }
     }
     store_mean<D>(acc, a.mean[tensor] + ((int64_t)bh * (tensor ? ca.nk : a.nb) + n) * D, lane);
   }
