@@ -32,10 +32,8 @@ constexpr int kKeyChunk = 64;    // keys staged per LDS chunk (one per lane)
 constexpr int kMaxPer = 64;      // max score columns per lane -> nk <= 4096
 
 __device__ __forceinline__ uint32_t order_key(float f) {
-  if (f != f) return 0u;       // NaN: below every number
-  if (f == 0.0f) f = 0.0f;     // -0.0 -> +0.0
-  const uint32_t u = __builtin_bit_cast(uint32_t, f);
-  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+  const uint32_t u = __builtin_bit_cast(uint32_t, f + 0.0f);  // -0.0 -> +0.0
+  return f != f ? 0u : u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);  // NaN: below every number
 }
 
 constexpr int kCompactCap = 512;  // compacted keys per wave (LDS words)
@@ -232,7 +230,7 @@ __global__ __launch_bounds__(256) void route_kernel(RouteArgs a) {
 #pragma unroll
       for (int e = 0; e < NPER; ++e) {
         const int col = e * 64 + lane;
-        sc[r][e] = (row < a.nq && col < a.nk) ? src[col] : 0.0f;
+        sc[r][e] = src[col < a.nk ? col : 0];  // wave_topk takes no column past nk
       }
     }
   } else {
@@ -472,6 +470,24 @@ __device__ __forceinline__ void tile_step_nf(const bf16x8 (&a)[3], const bf16x8 
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b0, acc, 0, 0, 0);
 }
 
+// A lane's 8 values of each k-step of its row, zero where there is no row: one
+// branch around all of the loads, so that none waits for another (one branch per
+// step made the fused routing 231 instead of 190 us at 32 heads x 900 x 900, 9.6
+// instead of 8.5 us at 2 x 32 x 32).
+template <int KST>
+__device__ __forceinline__ void load_row_steps(bool in, const float* src, f32x4 (&raw)[KST][2]) {
+#pragma unroll
+  for (int s = 0; s < KST; ++s) raw[s][0] = raw[s][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (in) {
+#pragma unroll
+    for (int s = 0; s < KST; ++s) {
+      raw[s][0] = *reinterpret_cast<const f32x4*>(src + 16 * s);
+      raw[s][1] = *reinterpret_cast<const f32x4*>(src + 16 * s + 4);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // The A pieces of 32 rows (row0 + lane % 32) for all k-steps: lane (r, g)
 // holds dims 16s + 8g .. + 8 of its row.  Rows at or past `nrows` (and
 // lanes whose row is not below `live`) are zero.
@@ -482,17 +498,13 @@ __device__ __forceinline__ bool load_row_pieces(const float* base, int row0, int
   const int r = lane % 32;
   const int row = row0 + r;
   const int g = lane / 32;
+  f32x4 raw[KST][2];
+  load_row_steps<KST>(r < live && row < nrows, base + (int64_t)row * D + 8 * g, raw);
   bool fin = true;
 #pragma unroll
   for (int s = 0; s < KST; ++s) {
-    f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
-    if (r < live && row < nrows) {
-      const float* src = base + (int64_t)row * D + 16 * s + 8 * g;
-      lo = *reinterpret_cast<const f32x4*>(src);
-      hi = *reinterpret_cast<const f32x4*>(src + 4);
-    }
-    fin = fin & all_finite8(lo, hi);
-    split8_wave(lo, hi, pa[s]);
+    fin = fin & all_finite8(raw[s][0], raw[s][1]);
+    split8_wave(raw[s][0], raw[s][1], pa[s]);
   }
   return __ballot(!fin) != 0;
 }
@@ -524,7 +536,8 @@ __global__ __launch_bounds__(64 * W) void select_mfma_kernel(RouteArgs a) {
   const bool a_bad = load_row_pieces<KST>(qb, row0, a.nq, D, QR, pa);
   const int ntiles = (a.nk + 31) / 32;
   for (int t = wave; t < ntiles; t += W) {
-    const int key = 32 * t + c;
+    f32x4 raw[KST][2];
+    load_row_steps<KST>(32 * t + c < a.nk, kb + (int64_t)(32 * t + c) * D + 8 * g, raw);
     f32x16 acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
@@ -532,12 +545,7 @@ __global__ __launch_bounds__(64 * W) void select_mfma_kernel(RouteArgs a) {
     // choice can be made per k-step.
 #pragma unroll
     for (int s = 0; s < KST; ++s) {
-      f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
-      if (key < a.nk) {
-        const float* src = kb + (int64_t)key * D + 16 * s + 8 * g;
-        lo = *reinterpret_cast<const f32x4*>(src);
-        hi = *reinterpret_cast<const f32x4*>(src + 4);
-      }
+      const f32x4 lo = raw[s][0], hi = raw[s][1];
       const bool b_bad = __ballot(!all_finite8(lo, hi)) != 0;
       bf16x8 pb[3];
       if (b_bad)
@@ -781,10 +789,11 @@ hipError_t launch_route(RouteArgs a, int BH, hipStream_t stream) {
 
 // One workgroup of 8 rows and 8 waves per CU at most, and one 32-key tile per
 // wave at most: routing is then one chain of loads, 48 MFMAs and a top-k, and one
-// launch instead of two.  Whole forward against scores + top-k, D = 128, fp16: 23.4
-// against 25.1 us at 2 heads x 32 blocks, 34.2 / 35.8 us at 8 x 64, 119.4 / 122.7 us
-// at 8 x 256; beyond the line 168.5 / 167.8 us at 5 x 400, 363 / 351 us at 2 x 900,
-// 114 / 106 us at 32 x 100.
+// launch instead of two.  Whole forward against scores + top-k, D = 128, fp16, when
+// the line was drawn: 23.4 / 25.1 us at 2 heads x 32 blocks, 34.2 / 35.8 us at 8 x 64,
+// 119.4 / 122.7 us at 8 x 256; beyond the line 168.5 / 167.8 us at 5 x 400, 363 / 351 us
+// at 2 x 900, 114 / 106 us at 32 x 100 (the fused kernel has since gained 1 us at the
+// small sizes, a fifth at the large ones, where it is still three times the two).
 bool select_short(int BH, int nq, int nk) { return nk <= 256 && (int64_t)BH * ((nq + 7) / 8) <= 256; }
 
 bool select_supported(int nk, int D) {
