@@ -13,7 +13,8 @@
 // registers.  The half tiles go through a ring of four LDS slots in the order
 // K(0), V(0), K(1), V(1), ..., each fetched three elements ahead.
 //   * Any text length: rows of the last half tile past the end re-read the last
-//     key (in bounds), their scores become -inf and their V rows zero in LDS.
+//     key (in bounds, and no maximum moves), their P and, in LDS, their V rows
+//     become zero.  (A masked score would be -inf * 0 at a scale of zero.)
 //   * Any query count: rows past the end repeat the last row and are not
 //     stored.
 //   * The softmax offset of a row is the maximum of its first half tile; where a
@@ -236,20 +237,20 @@ void text_attn_kernel(TextArgs p) {
     __syncthreads();
     if (more) dma(s + 1, 1, (2 * P + 3) % 4);
     qk(ring + 2 * P * kSlotBytes);
-    if (!more && tail) {
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (16 * kt + 4 * G + i >= tail) sacc[kt][qt][i] = -__builtin_inff();
-    }
     if (s == 0 && !exact) {
       m_run[0] = __builtin_elementwise_maximum(rowmax(0), kMinOffset);
       m_run[1] = __builtin_elementwise_maximum(rowmax(1), kMinOffset);
     }
-    const float l0 = exps(0), l1 = exps(1);
+    float l0 = exps(0), l1 = exps(1);
+    if (!more && tail) {
+#pragma unroll
+      for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (16 * (e / 4) + 4 * G + e % 4 >= tail) pf[qt][e] = from_f32<T>(0.0f);
+      l0 = Mfma<T>::sum8(pf[0], 0.0f);
+      l1 = Mfma<T>::sum8(pf[1], 0.0f);
+    }
     if (__ballot(!(l0 + l1 <= kMaxLaneSum))) dirty = true;  // wave-uniform, rare
     l_run[0] += l0;
     l_run[1] += l1;

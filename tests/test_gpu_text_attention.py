@@ -79,6 +79,17 @@ def test_offset_far_below_later_keys(device, dtype):
     _check(out, _reference(q, k, v, w, lens, D ** -0.5), dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("lens", [(31,), (32,), (33,), (40, 5), (64, 128)])
+def test_zero_scale_gives_the_mean_of_v(device, dtype, D, lens):
+    q, kv, w = _inputs(device, dtype, lens, 130, 2, D, seed=7)
+    k, v = kv[:, 0].transpose(0, 1), kv[:, 1].transpose(0, 1)
+    out = torch.empty_like(q)
+    text_attention(q.transpose(1, 2), k, v, lens, w, 1e-6, 0.0, out.transpose(1, 2))
+    _check(out, _reference(q, k, v, w, lens, 0.0), dtype)
+
+
 def test_non_finite_values(device):
     """Infinite scores and values act as in a softmax, and the text of the next
     item, which the last tile of an item reaches, never does."""
