@@ -18,8 +18,12 @@
 //   * Any query count: rows past the end repeat the last row and are not
 //     stored.
 //   * The softmax offset of a row is the maximum of its first half tile; where a
-//     later P sum passes 2^15 the workgroup walks the text again from the rows'
-//     exact maxima (rescaling O inside the walk spills 61 registers).
+//     later P sum passes 2^15 or is NaN (no score above -inf so far), or a row's
+//     whole sum is zero, the workgroup walks the text again from the rows' exact
+//     maxima (rescaling O inside the walk spills 61 registers).  P is there
+//     exp2((score - max) scale), as exact as the scores are at any size; the first
+//     walk's fma(score, scale, -offset) is off by the rounding of the offset, which
+//     a row shares until it overflows (|offset| of 2^28 and more).
 // Work ids run batch item fastest: items of different text lengths share an
 // XCD's time, and each XCD's heads keep their text K / V in its L2.
 //
@@ -37,7 +41,6 @@ namespace lcv {
 namespace {
 
 constexpr float kMaxLaneSum = 32768.0f;  // bound on a lane's P sum of one half tile: P stays a normal fp16 value
-constexpr float kMinOffset = -1e30f;     // offset of a row whose scores are all -inf so far
 
 struct TextArgs {
   TextAttn t;
@@ -192,14 +195,25 @@ void text_attn_kernel(TextArgs p) {
     mx = fmax3(mx, sacc[0][qt][3], sacc[1][qt][0]);
     mx = fmax3(mx, sacc[1][qt][1], sacc[1][qt][2]);
     mx = __builtin_elementwise_maximum(mx, sacc[1][qt][3]);
-    return max_quarters(mx) * sl2;
+    return max_quarters(mx);
   };
+  bool dirty = false, exact = false;
   auto exps = [&](int qt) {
+    if (exact) {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sacc[kt][qt][i] = (sacc[kt][qt][i] - m_run[qt]) * sl2;
+    } else {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sacc[kt][qt][i] = __builtin_fmaf(sacc[kt][qt][i], sl2, -m_run[qt]);
+    }
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        pf[qt][4 * kt + i] = from_f32<T>(fast_exp2(__builtin_fmaf(sacc[kt][qt][i], sl2, -m_run[qt])));
+      for (int i = 0; i < 4; ++i) pf[qt][4 * kt + i] = from_f32<T>(fast_exp2(sacc[kt][qt][i]));
     return Mfma<T>::sum8(pf[qt], 0.0f);
   };
   auto pv = [&](const uint8_t* Vs) {
@@ -228,7 +242,6 @@ void text_attn_kernel(TextArgs p) {
   // Half tile s: elements 2s (K, slot 2s mod 4) and 2s + 1 (V).  At the
   // barrier that starts an element every wave has consumed the one before, so
   // the element three ahead goes into its slot; at most two are in flight.
-  bool dirty = false, exact = false;
   auto run_half = [&](int s, auto par) {
     constexpr int P = decltype(par)::value;  // s mod 2
     const bool more = s + 1 < nh;
@@ -238,8 +251,8 @@ void text_attn_kernel(TextArgs p) {
     if (more) dma(s + 1, 1, (2 * P + 3) % 4);
     qk(ring + 2 * P * kSlotBytes);
     if (s == 0 && !exact) {
-      m_run[0] = __builtin_elementwise_maximum(rowmax(0), kMinOffset);
-      m_run[1] = __builtin_elementwise_maximum(rowmax(1), kMinOffset);
+      m_run[0] = rowmax(0) * sl2;
+      m_run[1] = rowmax(1) * sl2;
     }
     float l0 = exps(0), l1 = exps(1);
     if (!more && tail) {
@@ -272,11 +285,12 @@ void text_attn_kernel(TextArgs p) {
       run_half(s, Par<0>{});
       if (s + 1 < nh) run_half(s + 1, Par<1>{});
     }
+    if (__ballot(!(sum_quarters(l_run[0]) > 0.0f) || !(sum_quarters(l_run[1]) > 0.0f))) dirty = true;
     if (lane == 0) wave_dirty[wave] = dirty ? 1 : 0;
     __syncthreads();  // every ring read done (no DMA is outstanding here); flags visible
     if (exact || !(wave_dirty[0] | wave_dirty[1] | wave_dirty[2] | wave_dirty[3])) break;  // workgroup-uniform
     exact = true;
-    float mx[2] = {kMinOffset, kMinOffset};
+    float mx[2] = {-__builtin_inff(), -__builtin_inff()};
     for (int s = 0; s < nh; ++s) {  // the last key's repeats change no maximum
       dma(s, 0, 0);
       wait_vmcnt<0>();
@@ -296,8 +310,8 @@ void text_attn_kernel(TextArgs p) {
     if (nh > 1) dma(s0 + 1, 0, 2);
   }
 
-  // ---- Normalise, stage the rows in the ring, write whole rows.  A row with no
-  // finite score divides 0 by 0, as a softmax over it does.
+  // ---- Normalise, stage the rows in the ring, write whole rows.  A row whose
+  // scores are all -inf has a NaN sum, as a softmax over it does.
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
     const float inv = 1.0f / sum_quarters(l_run[qt]);

@@ -3,6 +3,8 @@ count) against fp32 torch on the rounded norms, and the layer's two routes."""
 
 from __future__ import annotations
 
+import math
+
 import pytest
 import torch
 
@@ -88,6 +90,25 @@ def test_zero_scale_gives_the_mean_of_v(device, dtype, D, lens):
     out = torch.empty_like(q)
     text_attention(q.transpose(1, 2), k, v, lens, w, 1e-6, 0.0, out.transpose(1, 2))
     _check(out, _reference(q, k, v, w, lens, 0.0), dtype)
+
+
+@pytest.mark.parametrize("lens", [(40,), (32,), (5, 70)])
+def test_scores_of_any_finite_size(device, lens):
+    """Every score near 1e31 or -1e31 (bf16 reaches it), all alike: the mean of v.
+    A row whose scores are all -inf has no softmax: NaN, as torch gives."""
+    N, H, D = 64, 1, 64
+    q, kv, _ = _inputs(device, torch.bfloat16, lens, N, H, D, seed=8)
+    q = torch.ones_like(q)
+    w = torch.ones(D, dtype=torch.bfloat16, device=device)
+    v = kv[:, 1].transpose(0, 1)
+    for value in (-1e30, 1e30, -1e10, float("-inf")):
+        k = torch.full_like(kv[:, 0], value).transpose(0, 1)
+        out = torch.empty_like(q)
+        text_attention(q.transpose(1, 2), k, v, lens, w, 1e-6, D ** -0.5, out.transpose(1, 2))
+        if math.isfinite(value):
+            _check(out, _reference(q, torch.zeros_like(k), v, w, lens, 1.0), torch.bfloat16)
+        else:
+            assert out.isnan().all()
 
 
 def test_non_finite_values(device):
