@@ -17,6 +17,7 @@ it; the cross-attention handles any batch with per-item text lengths.
 
 from __future__ import annotations
 
+import math
 from typing import Optional, Sequence
 
 import torch
@@ -324,11 +325,13 @@ class MultiHeadCrossAttention(nn.Module):
         return self._cross(x, cond, kv_seqlen)
 
     def _fusible(self, q, kv, lens) -> bool:
-        """Whether the text attention kernel takes these projections: 64-token
-        multiples always; any other lengths where nothing differentiates or
-        traces through the norms and the attention, and the lengths share out
-        text that is there."""
+        """Whether the text attention kernel takes these projections (at a scale
+        that it has): 64-token multiples always; any other lengths where nothing
+        differentiates or traces through the norms and the attention, and the
+        lengths share out text that is there."""
         if self.head_dim not in (64, 128) or not q.is_cuda or q.dtype not in (torch.float16, torch.bfloat16):
+            return False
+        if not 0.0 <= self.scale < math.inf:
             return False
         if q.shape[1] % 64 == 0 and all(n % 64 == 0 for n in lens):
             return True

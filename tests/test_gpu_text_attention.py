@@ -150,6 +150,19 @@ def test_layer_routes_agree(device, N, text):
         assert x.grad is not None
 
 
+@pytest.mark.parametrize("text", [(31, 33), (50, 9), (64, 128)])
+@pytest.mark.parametrize("scale", [0.0, -0.1])
+def test_layer_takes_any_scale(device, text, scale):
+    m = MultiHeadCrossAttention(256, 2, dtype=torch.float16, device=device)
+    m.scale = scale
+    x = torch.randn(2, 128, 256, device=device, dtype=torch.float16)
+    y = torch.randn(1, sum(text), 256, device=device, dtype=torch.float16)
+    with torch.no_grad():
+        got = m(x, y, text)
+        m.fused = False
+        _check(got, m(x, y, text).float(), torch.float16)
+
+
 def test_refused(device):
     q, kv, w = _inputs(device, torch.float16, (8, 8), 64, 2, 64, seed=1)
     k, v = kv[:, 0].transpose(0, 1), kv[:, 1].transpose(0, 1)
