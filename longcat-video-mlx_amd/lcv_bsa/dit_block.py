@@ -327,8 +327,8 @@ class MultiHeadCrossAttention(nn.Module):
     def _fusible(self, q, kv, lens) -> bool:
         """Whether the text attention kernel takes these projections (at a scale
         that it has): 64-token multiples always; any other lengths where nothing
-        differentiates or traces through the norms and the attention, and the
-        lengths share out text that is there."""
+        differentiates or traces through the norms and the attention, the
+        lengths share out text that is there and every row starts on 16 bytes."""
         if self.head_dim not in (64, 128) or not q.is_cuda or q.dtype not in (torch.float16, torch.bfloat16):
             return False
         if not 0.0 <= self.scale < math.inf:
@@ -338,7 +338,8 @@ class MultiHeadCrossAttention(nn.Module):
         n = lens[:q.shape[0]]
         return (len(n) == q.shape[0] and min(n) >= 1 and sum(n) <= kv.shape[1]
                 and plain_tensors(q, kv, self.q_norm.weight, self.k_norm.weight)
-                and q.data_ptr() % 16 == 0 and kv.data_ptr() % 16 == 0)
+                and all(t.data_ptr() % 16 == 0 and t.stride(-1) == 1
+                        and all(st >= self.head_dim and st % 8 == 0 for st in t.stride()[:-1]) for t in (q, kv)))
 
     def _cross_fused(self, q, kv, lens):
         """q [B, N, H, D], kv [1, L, 2, H, D]: k's norm, then q's norm and the

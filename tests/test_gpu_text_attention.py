@@ -163,6 +163,27 @@ def test_layer_takes_any_scale(device, text, scale):
         _check(got, m(x, y, text).float(), torch.float16)
 
 
+@pytest.mark.parametrize("part", ["q_linear", "kv_linear"])
+@pytest.mark.parametrize("pad", [4, 8])
+def test_layer_takes_projections_with_any_row_stride(device, part, pad):
+    class Padded(torch.nn.Module):
+        def __init__(self, linear):
+            super().__init__()
+            self.linear = linear
+
+        def forward(self, x):
+            return torch.nn.functional.pad(self.linear(x), (0, pad))[..., :-pad]
+
+    m = MultiHeadCrossAttention(256, 2, dtype=torch.float16, device=device)
+    setattr(m, part, Padded(getattr(m, part)))
+    x = torch.randn(2, 100, 256, device=device, dtype=torch.float16)
+    y = torch.randn(1, 59, 256, device=device, dtype=torch.float16)
+    with torch.no_grad():
+        got = m(x, y, (50, 9))
+        m.fused = False
+        _check(got, m(x, y, (50, 9)).float(), torch.float16)
+
+
 def test_refused(device):
     q, kv, w = _inputs(device, torch.float16, (8, 8), 64, 2, 64, seed=1)
     k, v = kv[:, 0].transpose(0, 1), kv[:, 1].transpose(0, 1)
