@@ -50,6 +50,14 @@ class RMSNorm_FP32(nn.Module):
         return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps)).to(x.dtype) * self.weight
 
 
+def plain_rms_norms(*norms: nn.Module) -> bool:
+    """Whether these are RMSNorm_FP32 and nothing else: no other class, forward or
+    hook, so that a kernel may do their work from ``weight`` and ``eps``."""
+    return (not torch.nn.modules.module._has_any_global_hook()
+            and all(type(m) is RMSNorm_FP32 and "forward" not in vars(m)
+                    and not m._forward_hooks and not m._forward_pre_hooks for m in norms))
+
+
 class LayerNorm_FP32(nn.Module):
     """LayerNorm computed in fp32, cast back to the input dtype (blocks.py:79-103)."""
 
@@ -222,9 +230,9 @@ class Attention(nn.Module, BSAAttention):
         return (out, cache) if return_kv else out
 
     def _cache_fusible(self, *tensors) -> bool:
-        """The norms around a KV cache as one kernel: nothing differentiates or
-        traces through them, and both round and weigh alike."""
-        return (self.q_norm.eps == self.k_norm.eps
+        """The norms around a KV cache as one kernel: they are plain, nothing
+        differentiates or traces through them, and both round and weigh alike."""
+        return (plain_rms_norms(self.q_norm, self.k_norm) and self.q_norm.eps == self.k_norm.eps
                 and plain_tensors(*tensors, self.q_norm.weight, self.k_norm.weight))
 
     def _continue_fused(self, q, k, v, x, shape, ncl, kv_cache):
@@ -326,9 +334,9 @@ class MultiHeadCrossAttention(nn.Module):
 
     def _fusible(self, q, kv, lens) -> bool:
         """Whether the text attention kernel takes these projections (at a scale
-        that it has): 64-token multiples always; any other lengths where nothing
-        differentiates or traces through the norms and the attention, the
-        lengths share out text that is there and every row starts on 16 bytes."""
+        that it has): 64-token multiples always; any other lengths where the norms
+        are plain, nothing differentiates or traces through them and the attention,
+        the lengths share out text that is there and every row starts on 16 bytes."""
         if self.head_dim not in (64, 128) or not q.is_cuda or q.dtype not in (torch.float16, torch.bfloat16):
             return False
         if not 0.0 <= self.scale < math.inf:
@@ -337,6 +345,7 @@ class MultiHeadCrossAttention(nn.Module):
             return True
         n = lens[:q.shape[0]]
         return (len(n) == q.shape[0] and min(n) >= 1 and sum(n) <= kv.shape[1]
+                and plain_rms_norms(self.q_norm, self.k_norm)
                 and plain_tensors(q, kv, self.q_norm.weight, self.k_norm.weight)
                 and all(t.data_ptr() % 16 == 0 and t.stride(-1) == 1
                         and all(st >= self.head_dim and st % 8 == 0 for st in t.stride()[:-1]) for t in (q, kv)))

@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import contextlib
 import os
 import sys
 from pathlib import Path
@@ -103,3 +104,40 @@ def wide_range_inputs(D: int, q_scale: float, dtype, seeds=(31, 32, 33), wide_ro
     idx = np.broadcast_to(np.arange(0, nb, 2, dtype=np.int32), (1, 2, nb, nb // 2)).copy()
     idx[0, 1] = idx[0, 1, :, ::-1]  # descending lists too
     return q.to(dtype), k.to(dtype), v.to(dtype), idx
+
+
+NORM_CHANGES = ("hook", "pre_hook", "global_hook", "forward", "subclass", "identity")
+
+
+@contextlib.contextmanager
+def changed_norms(what, layer):
+    """An attention layer's q_norm and k_norm made to do more, or other things,
+    than RMSNorm_FP32 does."""
+    import torch
+    from lcv_bsa.dit_block import RMSNorm_FP32
+
+    class Half(RMSNorm_FP32):
+        def forward(self, x):
+            return super().forward(x) / 2
+
+    handles = []
+    for name in ("q_norm", "k_norm"):
+        norm = getattr(layer, name)
+        if what == "hook":
+            handles.append(norm.register_forward_hook(lambda mod, args, out: out / 2))
+        elif what == "pre_hook":
+            handles.append(norm.register_forward_pre_hook(lambda mod, args: (args[0] + 1,)))
+        elif what == "forward":
+            norm.forward = lambda x: x / 2
+        elif what == "subclass":
+            norm.__class__ = Half
+        elif what == "identity":
+            setattr(layer, name, torch.nn.Identity())
+    if what == "global_hook":
+        handles.append(torch.nn.modules.module.register_module_forward_hook(
+            lambda mod, args, out: out / 2 if isinstance(mod, RMSNorm_FP32) else None))
+    try:
+        yield
+    finally:
+        for h in handles:
+            h.remove()

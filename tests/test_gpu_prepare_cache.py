@@ -8,6 +8,7 @@ import math
 
 import pytest
 import torch
+from conftest import NORM_CHANGES, changed_norms
 
 from lcv_bsa import mean_pool_blocks_3d, prepare_qk, prepare_qkv
 from lcv_bsa.block_ops import head_rms_norm
@@ -106,3 +107,27 @@ def test_layer_cache_with_and_without_gradients(device, dtype, policy, ncl):
         # a unit in the last place here and there, averaged out by the 2-norm
         assert (f.float() - s.float()).norm() <= eps * s.float().norm()
     assert math.isfinite(float(slow[1].float().sum()))
+
+
+@pytest.mark.parametrize("what", NORM_CHANGES)
+def test_layer_runs_its_norms_as_modules(device, what):
+    """Around a KV cache, hooks on the norms fire and another norm counts: the same
+    bits as with gradients, which torch's sequence gives."""
+    from lcv_bsa.dit_block import Attention
+
+    torch.manual_seed(4)
+    C, H, Hl, Wl, ncl, T = 256, 2, 8, 16, 2, 4
+    a = Attention(C, H, dtype=torch.float16, device=device)
+    a.enable_bsa, a.bsa_cond_noise, a.bsa_shape_policy = True, True, "contiguous"
+    x = torch.randn(1, (ncl + T) * Hl * Wl, C, dtype=torch.float16, device=device)
+    nc = ncl * Hl * Wl
+
+    def both():
+        out, cache = a(x[:, :nc], (ncl, Hl, Wl), return_kv=True)
+        return out, *cache, a.forward_with_kv_cache(x[:, nc:], (T, Hl, Wl), ncl, cache)
+
+    with changed_norms(what, a):
+        want = both()
+        with torch.no_grad():
+            got = both()
+    assert all(torch.equal(g, w) for g, w in zip(got, want))

@@ -7,6 +7,7 @@ import math
 
 import pytest
 import torch
+from conftest import NORM_CHANGES, changed_norms
 
 from lcv_bsa.block_ops import text_attention
 from lcv_bsa.dit_block import MultiHeadCrossAttention, RMSNorm_FP32
@@ -182,6 +183,18 @@ def test_layer_takes_projections_with_any_row_stride(device, part, pad):
         got = m(x, y, (50, 9))
         m.fused = False
         _check(got, m(x, y, (50, 9)).float(), torch.float16)
+
+
+@pytest.mark.parametrize("what", NORM_CHANGES)
+def test_layer_runs_its_norms_as_modules(device, what):
+    """Hooks on the norms fire and another norm counts, as in torch's sequence."""
+    m = MultiHeadCrossAttention(256, 2, dtype=torch.float16, device=device)
+    x = torch.randn(1, 100, 256, device=device, dtype=torch.float16)
+    y = torch.randn(1, 50, 256, device=device, dtype=torch.float16)
+    with torch.no_grad(), changed_norms(what, m):
+        got = m(x, y, (50,))
+        m.fused = False
+        assert torch.equal(got, m(x, y, (50,)))
 
 
 def test_refused(device):
