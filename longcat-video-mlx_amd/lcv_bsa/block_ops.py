@@ -115,7 +115,7 @@ def head_rms_norm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float = 
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """RMSNorm_FP32 over the last dim of a ``[B, H, S, D]`` view (any strides
     with dense D) into ``out`` (default: contiguous ``[B, H, S, D]``)."""
-    _require_device(x)
+    _require_device(x, *(t for t in (weight, out) if t is not None))
     B, H, S, D = x.shape
     if out is None:
         out = torch.empty((B, H, S, D), dtype=x.dtype, device=x.device)
@@ -150,7 +150,7 @@ def text_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, text_len: 
     text ``k`` (normalised), ``v`` ``[H, L, D]``: item b attends to the
     ``text_len[b]`` rows after those of the items before it.  Writes ``out``
     ``[B, H, N, D]`` (any strides with dense D)."""
-    _require_device(q, k, v, out)
+    _require_device(q, k, v, out, q_weight)
     B, H, N, D = q.shape
     L = k.shape[1]
     if tuple(k.shape) != (H, L, D) or tuple(v.shape) != (H, L, D) or tuple(out.shape) != (B, H, N, D):

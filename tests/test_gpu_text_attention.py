@@ -9,7 +9,8 @@ import pytest
 import torch
 from conftest import NORM_CHANGES, changed_norms
 
-from lcv_bsa.block_ops import text_attention
+from lcv_bsa.block_ops import head_rms_norm, text_attention
+from lcv_bsa.block_sparse_attention import BSADeviceError
 from lcv_bsa.dit_block import MultiHeadCrossAttention, RMSNorm_FP32
 
 pytestmark = pytest.mark.gpu
@@ -204,3 +205,13 @@ def test_refused(device):
     for lens in [(8, 9), (0, 8), (8,), (16, -1)]:
         with pytest.raises(ValueError):
             text_attention(q.transpose(1, 2), k, v, lens, w, 1e-6, 0.125, out)
+
+
+def test_tensors_on_the_host_are_refused(device):
+    q, kv, w = _inputs(device, torch.float16, (8, 8), 64, 2, 64, seed=1)
+    k, v = kv[:, 0].transpose(0, 1), kv[:, 1].transpose(0, 1)
+    with pytest.raises(BSADeviceError):
+        text_attention(q.transpose(1, 2), k, v, (8, 8), w.cpu(), 1e-6, 0.125, torch.empty_like(q).transpose(1, 2))
+    for kw in (dict(weight=w.cpu()), dict(weight=w, out=torch.empty(2, 2, 64, 64, dtype=torch.float16))):
+        with pytest.raises(BSADeviceError):
+            head_rms_norm(q.transpose(1, 2), **kw)
