@@ -21,7 +21,16 @@ import torch
 from . import _lib
 from .block_sparse_attention import _dtype_code, _require_device, _stream, _strides
 
-__all__ = ["residual_norm", "swiglu", "head_rms_norm", "adaln_modulation", "text_attention", "plain_tensors"]
+__all__ = ["residual_norm", "swiglu", "head_rms_norm", "adaln_modulation", "text_attention", "plain_tensors",
+           "unwatched"]
+
+
+def unwatched(*ts: torch.Tensor) -> bool:
+    """No transform, trace or tensor subclass looks on what torch does with ``ts``."""
+    if (torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0):
+        return False
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in ts)
 
 
 def plain_tensors(*ts: Optional[torch.Tensor]) -> bool:
@@ -35,11 +44,7 @@ def plain_tensors(*ts: Optional[torch.Tensor]) -> bool:
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
         return False
-    if (torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0):
-        return False
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == t0.dtype and t.device == t0.device
-               for t in ts)
+    return unwatched(*ts) and all(t.dtype == t0.dtype and t.device == t0.device for t in ts)
 
 
 def _ptr(t: Optional[torch.Tensor]):

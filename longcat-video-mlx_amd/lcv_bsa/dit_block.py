@@ -25,7 +25,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .attention import BSAAttention, dense_attention, validate_backend
-from .block_ops import adaln_modulation, head_rms_norm, plain_tensors, residual_norm, swiglu, text_attention
+from .block_ops import adaln_modulation, head_rms_norm, plain_tensors, residual_norm, swiglu, text_attention, unwatched
 from .block_sparse_attention import bsa_attention
 from .prepare import prepare_qk, prepare_qkv
 from .rope_3d import rope_3d
@@ -405,7 +405,7 @@ class LongCatSingleStreamBlock(nn.Module):
         (longcat_video_dit.py:80-138); on the fused path one kernel."""
         lin = self.adaLN_modulation[1]
         w, b = lin.weight, lin.bias
-        if (fused and t.dim() == 3 and t.is_cuda and w.device == b.device == t.device
+        if (fused and t.dim() == 3 and t.is_cuda and w.device == b.device == t.device and unwatched(t, w, b)
                 and w.dtype == b.dtype and w.dtype in (torch.float16, torch.bfloat16)
                 and w.data_ptr() % 16 == 0 and w.is_contiguous() and w.shape[0] == 6 * self.hidden_size
                 and t.shape[-1] == w.shape[1] <= 1024 and w.shape[1] % 8 == 0

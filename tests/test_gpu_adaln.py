@@ -39,3 +39,21 @@ def test_block_modulation_routes_agree(device, K):
         for got, want in zip(blk._modulation(t, True), blk._modulation(t, False), strict=True):
             assert got.shape == want.shape == (2, 5, 1, 256) and got.dtype == torch.float32
             assert torch.allclose(got, want, rtol=1e-5, atol=2e-6)
+
+
+def test_a_weight_that_stands_for_others(device):
+    """A tensor subclass says itself what its values are: only torch asks it."""
+    class Doubled(torch.Tensor):
+        def float(self):
+            return 2 * self.as_subclass(torch.Tensor).float()
+
+    blk = LongCatSingleStreamBlock(256, 2, 4, 64, dtype=torch.float16, device=device)
+    lin = blk.adaLN_modulation[1]
+    t = torch.randn(2, 5, 64, device=device)
+    with torch.no_grad():
+        for name in ("weight", "bias"):
+            doubled = getattr(lin, name).detach().as_subclass(Doubled)
+            delattr(lin, name)
+            setattr(lin, name, doubled)
+            for got, want in zip(blk._modulation(t, True), blk._modulation(t, False), strict=True):
+                assert torch.allclose(got, want, rtol=1e-5, atol=2e-6)
