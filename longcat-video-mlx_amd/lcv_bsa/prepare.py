@@ -22,6 +22,7 @@ here with the reference's angle formula (rope_3d.py:65-93).
 
 from __future__ import annotations
 
+import threading
 from typing import Optional, Sequence
 
 import torch
@@ -46,7 +47,9 @@ def _axis_table(dim: int, n: int, device) -> tuple[torch.Tensor, torch.Tensor]:
 
 
 _TABLES: dict = {}
-_MAX_TABLES = 256  # of at most 48 KB; none is dropped, so a kernel in flight keeps the one it reads
+_TABLES_LOCK = threading.Lock()
+_MAX_TABLE_BYTES = 256 << 20  # about 10,000 tables of a 720p grid
+_table_bytes = 0              # held now
 
 
 def rope_table(head_dim: int, grid: Sequence[int], device=None) -> torch.Tensor:
@@ -56,24 +59,33 @@ def rope_table(head_dim: int, grid: Sequence[int], device=None) -> torch.Tensor:
     Built once per (head_dim, grid, device) and kept: the kernel only reads
     it, and building it takes about thirty small launches (~0.15 ms at
     720p), which would otherwise recur in every attention layer.  A table is
-    complete before it is kept, so that any stream may read it; one built under
-    stream capture belongs to that graph and is not kept."""
+    complete before it is kept, so that any stream may read it, and none is
+    dropped, so that a kernel in flight or in a graph keeps the one it reads.
+    Once 256 MiB are held, further ones are built for the caller's stream alone,
+    without a wait; so is one built under stream capture, which belongs to that
+    graph."""
+    global _table_bytes
     dev = torch.device(device) if device is not None else torch.device("cpu")
     if dev.type == "cuda" and dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
     key = (int(head_dim), tuple(int(x) for x in grid), dev)
     table = _TABLES.get(key)
-    if table is None:
-        table = _build_table(head_dim, grid, dev)
-        if dev.type == "cuda":
-            stream = torch.cuda.current_stream(dev)
-            with torch.cuda.device(dev):
-                if torch.cuda.is_current_stream_capturing():
-                    return table
-            stream.synchronize()
-        if len(_TABLES) < _MAX_TABLES:
+    if table is not None:
+        return table
+    table = _build_table(head_dim, grid, dev)
+    size = table.numel() * table.element_size()
+    if _table_bytes + size > _MAX_TABLE_BYTES:
+        return table
+    if dev.type == "cuda":
+        with torch.cuda.device(dev):
+            if torch.cuda.is_current_stream_capturing():
+                return table
+        torch.cuda.current_stream(dev).synchronize()
+    with _TABLES_LOCK:
+        if key not in _TABLES and _table_bytes + size <= _MAX_TABLE_BYTES:
             _TABLES[key] = table
-    return table
+            _table_bytes += size
+        return _TABLES.get(key, table)
 
 
 def _build_table(head_dim: int, grid: Sequence[int], device) -> torch.Tensor:

@@ -554,3 +554,18 @@ def test_gathered_reference_matches_oracle():
     assert np.abs(got - ref).max() < 2e-5
     wrong = gathered_attention_fp32(q, kk.transpose(2, 3).reshape(B, H, S, D), v, idx, 0.3).numpy()
     assert np.abs(wrong - ref).max() > 1e-2
+
+
+def test_rope_tables_are_kept_up_to_a_bound(monkeypatch):
+    from lcv_bsa import prepare as P
+
+    monkeypatch.setattr(P, "_TABLES", {})
+    monkeypatch.setattr(P, "_table_bytes", 0, raising=False)
+    grids = [(1, 1, n) for n in range(1, 301)]
+    tables = [P.rope_table(64, g) for g in grids]
+    assert all(P.rope_table(64, g) is t for g, t in zip(grids, tables))
+    held = sum(t.numel() for t in tables) * 4
+    monkeypatch.setattr(P, "_MAX_TABLE_BYTES", held, raising=False)
+    first, again = P.rope_table(64, (2, 1, 1)), P.rope_table(64, (2, 1, 1))
+    assert first is not again and torch.equal(first, again) and len(P._TABLES) == 300
+    assert P.rope_table(64, grids[0]) is tables[0]

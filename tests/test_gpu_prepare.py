@@ -130,3 +130,72 @@ def test_prepare_rejects_bad_arguments(device):
     with pytest.raises(ValueError, match="norm weight"):
         prepare_qk(q, k, (8, 8, 16), q_weight=torch.ones(64, device=device), shape=(8, 8, 16),
                    chunk_thw=(4, 4, 4))
+
+
+def _table_inputs(device, seed=0):
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    return tuple(torch.randn(1, 2, 192, 64, generator=g).to(device, torch.float16) for _ in range(2))
+
+
+def _prepared(qk, grid):
+    from lcv_bsa import prepare_qk
+
+    return prepare_qk(*qk, grid, shape=(1, 1, 192), chunk_thw=(1, 1, 64))
+
+
+def test_rope_table_beyond_the_bound_needs_no_wait(device, monkeypatch):
+    from lcv_bsa import prepare as P
+
+    qk = _table_inputs(device)
+    want = _prepared(qk, (1, 3, 64))
+    waits = []
+    monkeypatch.setattr(torch.cuda.Stream, "synchronize", lambda self: waits.append(self))
+    monkeypatch.setattr(P, "_TABLES", {})
+    monkeypatch.setattr(P, "_MAX_TABLE_BYTES", 0)
+    for _ in range(2):
+        got = _prepared(qk, (1, 3, 64))
+        assert all(torch.equal(g, w) for g, w in zip(got, want))
+    assert not waits and not P._TABLES
+
+
+def test_rope_table_is_complete_for_every_stream(device, monkeypatch):
+    """Built behind other work on one stream, read on another at once."""
+    from lcv_bsa import prepare as P
+
+    want = P._build_table(64, (1, 2, 96), device)
+    torch.cuda.synchronize()
+    monkeypatch.setattr(P, "_TABLES", {})
+    a, b = torch.cuda.Stream(device=device), torch.cuda.Stream(device=device)
+    with torch.cuda.stream(a):
+        x = torch.ones(4096, 4096, device=device)
+        for _ in range(20):
+            x = x @ x / 4096  # some milliseconds
+        P.rope_table(64, (1, 2, 96), device)
+    with torch.cuda.stream(b):
+        got = P.rope_table(64, (1, 2, 96), device).clone()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+
+
+def test_rope_table_of_a_captured_call_stays_with_its_graph(device, monkeypatch):
+    """A grid first met under capture: its table is not kept, the graph's replays
+    and an eager call in between give the same bits."""
+    from lcv_bsa import prepare as P
+
+    monkeypatch.setattr(P, "_TABLES", {})
+    qk = _table_inputs(device)
+    _prepared(qk, (1, 1, 192))  # warm up on another grid
+    grid = (3, 1, 64)
+    torch.cuda.synchronize()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream(device=device)
+    with torch.cuda.graph(graph, stream=side):
+        out = _prepared(qk, grid)
+    assert (64, grid, device) not in P._TABLES
+    for seed in range(1, 5):
+        for t, new in zip(qk, _table_inputs(device, seed)):
+            t.copy_(new)
+        graph.replay()
+        want = _prepared(qk, grid)
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, w) for o, w in zip(out, want))
+    assert (64, grid, device) in P._TABLES
