@@ -3,9 +3,10 @@
 //
 // Same semantics as the kernels of attn_fwd.hip (softmax over the listed
 // blocks only; longcat_video/models/block_sparse_attention.py:201-250).  An
-// fp32 value x is split exactly into three bf16 pieces, x = p0 + p1 + p2, each
-// the round-to-nearest of what the previous ones leave (|p1| <= 2^-8 |x|,
-// |p2| <= 2^-16 |x|), and a product x y is formed from the six piece products
+// fp32 value x of 2^-103 and more in size, or zero, is split exactly into three
+// bf16 pieces, x = p0 + p1 + p2, each the round-to-nearest of what the previous
+// ones leave (|p1| <= 2^-8 |x|, |p2| <= 2^-16 |x|; smaller values are seen to
+// below, at kMinExact), and a product x y is formed from the six piece products
 // p_i q_j with i + j <= 2: each is exact in fp32 and the dropped ones are
 // below 2^-23 |x y| together, less than one fp32 rounding.  Six
 // 16 x 16 x 32 bf16 MFMAs cost 96 matrix cycles where the eight fp32 MFMAs of
@@ -21,10 +22,26 @@
 // cycles, the VALU (a third of it splitting K and V tiles) 32 %, LDS 29 %, with
 // no bank conflicts: what bounds it is how little the two or three workgroups of
 // a CU overlap these, and the last generation of workgroups.
+#include <algorithm>
+
 #include "attn_common.h"
 
 namespace lcv {
 namespace {
+
+// A value of at least kMinExact (or zero) has three pieces that are normal bf16
+// numbers or zero, so nothing is cut off it: 2^-103 less 23 bits is 2^-126.
+//   V: a smaller value, anywhere in the tiles, sends the workgroup to the second
+//      walk.
+//   P lies in [2^-149, 1]; scaled by 2^32 (exact, and divided out with the row sum)
+//      its normal values are above the line, and O stays finite for |V| < 2^77.
+//   Q: as V, and so does |q scale| >= kMaxQ.  Below that, what is cut off K (below
+//      2^-126 a value) moves no score by more than D 2^-126 kMaxQ <= 2^-29.
+constexpr float kMinExact = 0x1p-103f, kPScale = 0x1p32f, kMaxQ = 0x1p90f;
+
+// 2 |x| as an integer less one: of nonzero values the order of |x|, zero the largest.
+__device__ __forceinline__ uint32_t size_key(float x) { return (__builtin_bit_cast(uint32_t, x) << 1) - 1u; }
+constexpr uint32_t kMinExactKey = (__builtin_bit_cast(uint32_t, kMinExact) << 1) - 1u;
 
 // Pieces of a pair of fp32 values: w[i] holds piece i of x0 (low half) and x1.
 __device__ __forceinline__ void split2(float x0, float x1, uint32_t (&w)[3]) {
@@ -127,8 +144,8 @@ struct F32Occupancy {
 //
 // Values that the split cannot carry (inf, NaN, or so close to the fp32
 // maximum that they round to a bf16 infinity) turn their row's O into a NaN;
-// a workgroup that ends with a non-finite O or row sum walks again on the
-// vector ALU, whose result stands.
+// a workgroup that ends with a non-finite O or row sum, or met a value below
+// kMinExact where that counts, walks again on the vector ALU, whose result stands.
 template <int D>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(F32Occupancy<D>::kWaves, F32Occupancy<D>::kWaves)))
@@ -171,9 +188,11 @@ void attn_f32_kernel(AttnParams p) {
   // Q^T pieces: qf[i][ks] holds piece i of query 16 wave + gi, D 32 ks + 8 G .. + 7.
   const int32_t qtok = block_base_token(p.g, qb) + voxel_row_offset(p.g, 16 * wave + gi);
   bf16x8 qf[3][D / 32];
+  uint32_t least = ~0u;  // least size_key of the Q and V values this thread split; 0: Q or scale too large
   {
     const float* qrow = qbase + (int64_t)qtok * p.q_ss + 8 * G;
     f32x4 raw[D / 32][2];
+    float q_max = 1.0f;
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) {
       raw[ks][0] = *reinterpret_cast<const f32x4*>(qrow + 32 * ks);
@@ -186,7 +205,13 @@ void attn_f32_kernel(AttnParams p) {
       split8(raw[ks][0], raw[ks][1], pc);
 #pragma unroll
       for (int i = 0; i < 3; ++i) qf[i][ks] = pc[i];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        least = std::min(least, size_key(raw[ks][i / 4][i % 4]));
+        q_max = fmaxf(q_max, __builtin_fabsf(raw[ks][i / 4][i % 4]));
+      }
     }
+    if (!(q_max * __builtin_fabsf(p.scale_log2) < kMaxQ)) least = 0;
   }
 
   // Tile staging: task u of a thread is float4 c4 of row r0 + kStep u of the
@@ -309,11 +334,16 @@ void attn_f32_kernel(AttnParams p) {
     }
     f32x4 pe[2];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) pe[e / 4][e % 4] = fast_exp2(s[e] - m_run);
+    for (int e = 0; e < 8; ++e) pe[e / 4][e % 4] = fast_exp2(s[e] - m_run) * kPScale;
     l_run += ((pe[0][0] + pe[0][1]) + (pe[0][2] + pe[0][3])) + ((pe[1][0] + pe[1][1]) + (pe[1][2] + pe[1][3]));
     bf16x8 pf[3];
     split8(pe[0], pe[1], pf);
     store_tile(vst, Vp, vw0, 0);
+#pragma unroll
+    for (int u = 0; u < kTasks; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; i += 2)
+        least = std::min(std::min(least, size_key(vst[u][i])), size_key(vst[u][i + 1]));
     __syncthreads();
     if (jn < p.top_k) load_k(tokn, halfn);
 
@@ -349,7 +379,7 @@ void attn_f32_kernel(AttnParams p) {
   for (int dt = 0; dt < D / 16; ++dt)
 #pragma unroll
     for (int i = 0; i < 4; ++i) probe = fmaf(o[dt][i], 0.0f, probe);
-  if (__syncthreads_or(!(probe == 0.0f))) {
+  if (__syncthreads_or(least < kMinExactKey || !(probe == 0.0f))) {
     slow_walk<D>(p, bh, qb, qbase, kbase, vbase, obase);
     return;
   }

@@ -110,3 +110,40 @@ def test_values_the_split_cannot_carry(device, D, where, value):
     assert not fin.all() or value == 3.402e38
     assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got[got.isinf()], ref[ref.isinf()])
     assert torch.allclose(got[fin], ref[fin], rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("what", ["small v", "a small column of v", "subnormal v", "small q, large k",
+                                  "small k, large q", "small k, large scale", "weights near underflow, large v"])
+def test_values_far_from_one(device, D, what):
+    """Values whose bf16 pieces reach the subnormal range keep every bit that the
+    vector-ALU kernel keeps.  Each small value is made of 24 significant bits."""
+    S, top_k = 512, 3
+    q, k, v, idx = _inputs(device, 1, D, S, S, 8, 8, top_k, seed=11)
+    scale = D ** -0.5
+    if what == "small v":
+        v = v * 2.0 ** -118
+    elif what == "a small column of v":
+        v[..., 7] *= 2.0 ** -120
+    elif what == "subnormal v":
+        v = v * 2.0 ** -100 * 2.0 ** -30
+    elif what == "small q, large k":
+        q, k = q * 2.0 ** -116, k * 2.0 ** 116
+    elif what == "small k, large q":
+        q, k = q * 2.0 ** 118, k * 2.0 ** -118
+    elif what == "small k, large scale":
+        k, scale = k * 2.0 ** -118, scale * 2.0 ** 118
+    else:  # exp2 of about -117 against values of 2^115
+        q.zero_()
+        q[..., 0] = 1.0
+        k[..., 0] = torch.where(torch.arange(S, device=device) % 64 == 5, -81.0, 0.0)
+        v = v * torch.where(torch.arange(S, device=device) % 64 == 5, 2.0 ** 115, 2.0 ** -6)[:, None]
+        scale = 1.0
+    kw = dict(chunk_thw=(1, 1, 64), shape=(1, 1, S), sm_scale=scale)
+    got = bsa_attention_hip(q, k, v, idx, **kw).double().cpu()
+    valu = bsa_attention_hip(_unaligned(q), _unaligned(k), _unaligned(v), idx, **kw).double().cpu()
+    tok = _tokens((1, 1, S), (1, 1, 64))
+    ref = _exact(q, k, v, idx, tok, tok, scale)
+    # Column by column: a small one counts as much as the others.
+    err, err_valu = ((x - ref).norm(dim=-2) / ref.norm(dim=-2) for x in (got, valu))
+    assert (err <= torch.clamp(1.25 * err_valu, min=2e-6)).all(), ((err / err_valu).max(), err.max())
