@@ -211,7 +211,7 @@ hipError_t launch_schedule(const int32_t* idx, int BH, int nq, int nk, int top_k
                            hipStream_t stream);
 bool schedule_supported(int nq, int nk);
 // Whether the launch order saves the attention more than its sort costs.
-bool schedule_pays(int nk);
+bool schedule_pays(int BH, int nq, int nk);
 
 // Fused RMSNorm + 3D RoPE + block means of q and k (fp16/bf16, D 64/128).
 // The RoPE table holds cos and sin per axis: [rT*dt/2 | rT*dt/2 | rH*dh/2 |

@@ -392,7 +392,8 @@ int run_forward(const void* q, const void* k, const void* v, int dtype, int64_t 
                        what);
   }
   if (st) return st;
-  const bool sched = lcv::schedule_supported((int)nb, (int)nk) && lcv::schedule_pays((int)nk);
+  const bool sched =
+      lcv::schedule_supported((int)nb, (int)nk) && lcv::schedule_pays((int)(B * H), (int)nb, (int)nk);
   if (sched) {
     snprintf(what, sizeof(what), "%s(schedule)", name);
     st = launch_status(lcv::launch_schedule(idx, (int)(B * H), (int)nb, (int)nk, (int)top_k, order,

@@ -1,10 +1,11 @@
-// Launch order of the q-blocks of each head for the attention kernel, for heads
-// of more than 320 K/V blocks (schedule_pays).
+// Launch order of the q-blocks of each head for the attention kernel, at all but
+// small sizes (schedule_pays).
 //
-// Any order gives the same results up to fp32 rounding: each q-block is
-// computed by one workgroup from its own routing list, and its launch slot
-// sets where its walk over that list starts (the summation order).  For a
-// given order the result is deterministic.  The order matters for the L2: each
+// Any order gives the same results up to rounding: each q-block is computed by
+// one workgroup from its own routing list, and its launch slot sets where its
+// walk over that list starts: the order of the sums, and the offset that a 16-bit
+// P is rounded against, so that a 16-bit output may differ by a unit in the last
+// place (its error against 64 bits does not).  For a given order the result is deterministic.  The order matters for the L2: each
 // workgroup walks its KV blocks in ascending order, so workgroups that run at
 // the same time on an XCD re-read each other's K/V tiles from L2 when their
 // lists start at nearby blocks.  Sorting the q-blocks of a head by
@@ -157,13 +158,15 @@ bool schedule_supported(int nq, int nk) {
   return nq >= 1 && nq <= kMaxSched && nk >= 1 && nk <= kMaxKvBlocks;
 }
 
-// The order groups q-blocks that read the same K/V blocks: it pays once a head's
-// blocks outgrow what the resident workgroups share anyway.  Whole forward with one
-// sixteenth of the blocks kept, without against with the order: 92.4 / 96.7 us at 32
-// heads x 90 blocks of 64 x 128 fp16, 319.6 / 324.6 us at 225, 531 / 541 us at 312, then
-// 1,034 / 1,027 us at 450 and 306 / 297 us at 2 heads x 900 (D = 64: 311 / 315 us at
-// 320, equal at 450 to 900; fp32: 316 / 320 us at 8 heads x 195 blocks).
-bool schedule_pays(int nk) { return nk > 320; }
+// The order groups q-blocks that read the same K/V blocks.  Its sort costs 2 to 4 us,
+// which it does not earn back where the workgroups are four generations of the six
+// that a CU holds at most and a head's blocks are few.  Whole forward with one
+// sixteenth of the blocks kept, D = 128, without against with the order: 60.0 / 63.8 us
+// at 1 head x 320 blocks, 91.4 / 95.2 at 32 x 90, 155 / 158 at 8 x 320, 172 / 175 at
+// 32 x 160, 198 / 201 at 32 x 168, 224 / 225 at 32 x 182; D = 64 142 / 144 at 32 x 192;
+// fp32 129 / 132 at 8 x 128, 248 / 247 at 16 x 128.  Beyond the line 321 / 321 us at
+// 32 x 225, 427 / 428 at 32 x 273 voxels, 842 / 835 at 64 x 273, 306 / 297 at 2 x 900.
+bool schedule_pays(int BH, int nq, int nk) { return nk > 320 || (int64_t)BH * nq > 6144; }
 
 hipError_t launch_schedule(const int32_t* idx, int BH, int nq, int nk, int top_k, int32_t* order,
                            hipStream_t stream) {

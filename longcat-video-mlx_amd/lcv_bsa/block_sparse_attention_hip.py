@@ -29,7 +29,8 @@ __all__ = [
 ]
 
 MAX_SCHEDULED_BLOCKS = 4096
-MIN_KV_BLOCKS_SCHEDULED = 321  # below, the sort costs what the order saves (schedule_pays in csrc/schedule.hip)
+# Up to both, the sort costs what the order saves (schedule_pays in csrc/schedule.hip).
+UNSCHEDULED_KV_BLOCKS, UNSCHEDULED_WORKGROUPS = 320, 6144
 
 
 def schedule_block_order(block_indices: torch.Tensor, num_kv_blocks: Optional[int] = None) -> torch.Tensor:
@@ -129,7 +130,8 @@ def bsa_attention_hip(
     if code != _lib.F32:
         q, k, v = _aligned_rows(q), _aligned_rows(k), _aligned_rows(v)
     nk = num_blocks(kshape, chunk_thw)
-    order = schedule_block_order(bi, nk) if nb <= MAX_SCHEDULED_BLOCKS and nk >= MIN_KV_BLOCKS_SCHEDULED else None
+    pays = nk > UNSCHEDULED_KV_BLOCKS or B * H * nb > UNSCHEDULED_WORKGROUPS
+    order = schedule_block_order(bi, nk) if nb <= MAX_SCHEDULED_BLOCKS and pays else None
     out = _output(out, q)
     st = _lib.load().lcv_bsa_attn_fwd_kv(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), code, B, H, S, Sk, D,

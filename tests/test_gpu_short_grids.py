@@ -18,10 +18,27 @@ def _qkv(device, dtype, H, nq, nk, D, seed):
     return tuple(torch.randn(1, H, 64 * n, D, generator=g).to(device, dtype) for n in (nq, nk, nk))
 
 
+def _attend(q, k, v, idx, nq, nk, order):
+    """The attention stage alone, in the launch order given."""
+    from lcv_bsa import _lib
+    from lcv_bsa.block_sparse_attention import _dtype_code, _geom, _stream, _strides
+
+    out, (_, H, S, D) = torch.empty_like(q), q.shape
+    st = _lib.load().lcv_bsa_attn_fwd_kv(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _dtype_code(q), 1, H, S, k.shape[2], D, _strides(q), _strides(k),
+        _strides(v), idx.data_ptr(), None if order is None else order.data_ptr(), idx.shape[-1], D ** -0.5,
+        _geom((1, 1, 64 * nq), (1, 1, 64)), _geom((1, 1, 64 * nk), (1, 1, 64)), out.data_ptr(), _strides(out),
+        _stream(q))
+    _lib.check(st, "attn_fwd_kv")
+    return out
+
+
 # (H, q-blocks, k-blocks): one block, one key tile and one past it, the widest
-# fused row, the last and first grids of 256 workgroups, and 320 / 321 blocks.
+# fused row, the last and first grids of 256 workgroups, 320 / 321 blocks, and
+# 6,144 / 6,150 attention workgroups.
 GRIDS = [(1, 1, 1), (2, 32, 32), (2, 33, 33), (1, 256, 256), (1, 257, 257), (8, 256, 256), (9, 256, 256),
-         (3, 7, 255), (1, 320, 320), (1, 321, 321), (2, 64, 321), (4, 1, 40)]
+         (3, 7, 255), (1, 320, 320), (1, 321, 321), (2, 64, 321), (4, 1, 40),
+         (24, 256, 256), (25, 246, 246)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
@@ -62,3 +79,16 @@ def test_pool_of_two_grids_in_one_launch(device):
     out, idx = bsa_attention(q, k, v, shape, **kw)
     want, widx = bsa_attention(q, k, v, shape, block_means=means, **kw)
     assert torch.equal(idx, widx) and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("H,nq,nk,ordered", [(24, 256, 320, False), (25, 246, 320, True), (24, 200, 321, True)])
+def test_order_is_left_out_of_small_grids_only(device, H, nq, nk, ordered):
+    """Beyond the line the forward gives the bits of the ordered stages."""
+    q, k, v = _qkv(device, torch.bfloat16, H, nq, nk, 64, seed=nk)
+    shape, kv_shape, chunk = (1, 1, 64 * nq), (1, 1, 64 * nk), (1, 1, 64)
+    out, idx = bsa_attention(q, k, v, shape, chunk_thw=chunk, top_k=20, return_indices=True, kv_shape=kv_shape)
+    want = _attend(q, k, v, idx, nq, nk, schedule_block_order(idx, nk) if ordered else None)
+    assert torch.equal(out, want)
+    other = _attend(q, k, v, idx, nq, nk, None if ordered else schedule_block_order(idx, nk))
+    assert not torch.equal(out, other)  # another order of the sums
+    assert (out.float() - other.float()).norm() <= 2.0 ** -8 * out.float().norm()
