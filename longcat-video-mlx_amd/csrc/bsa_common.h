@@ -172,7 +172,7 @@ hipError_t launch_select(const float* qbar, const float* kbar, int B, int H, int
                          int nk, int D, int top_k, int32_t* idx, hipStream_t stream);
 bool select_supported(int nk, int D);
 // Whether the fused select beats score GEMM + top-k.
-bool select_short(int BH, int nq, int nk);
+bool select_short(int BH, int nq, int nk, int D);
 
 struct AttnParams {
   const void* q;

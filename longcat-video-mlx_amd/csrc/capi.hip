@@ -369,7 +369,7 @@ int run_forward(const void* q, const void* k, const void* v, int dtype, int64_t 
                        what);
     if (st) return st;
   }
-  if (score && !lcv::select_short((int)(B * H), (int)nb, (int)nk)) {
+  if (score && !lcv::select_short((int)(B * H), (int)nb, (int)nk, (int)D)) {
     // Slices [c0, c0 + n) of the B*H (b, h) pairs; the scores of one slice
     // are read by its top-k before the next slice's GEMM rewrites them (one
     // stream).

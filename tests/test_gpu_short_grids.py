@@ -34,11 +34,11 @@ def _attend(q, k, v, idx, nq, nk, order):
 
 
 # (H, q-blocks, k-blocks): one block, one key tile and one past it, the widest
-# fused row, the last and first grids of 256 workgroups, 320 / 321 blocks, and
+# fused rows, the last and first grids of 256 workgroups, 320 / 321 blocks, and
 # 6,144 / 6,150 attention workgroups.
 GRIDS = [(1, 1, 1), (2, 32, 32), (2, 33, 33), (1, 256, 256), (1, 257, 257), (8, 256, 256), (9, 256, 256),
          (3, 7, 255), (1, 320, 320), (1, 321, 321), (2, 64, 321), (4, 1, 40),
-         (24, 256, 256), (25, 246, 246)]
+         (24, 256, 256), (25, 246, 246), (8, 192, 192), (2, 193, 193), (11, 190, 190), (8, 3, 192)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
@@ -56,6 +56,15 @@ def test_forward_matches_stages(device, dtype, D, H, nq, nk):
     for kw in ({}, {"block_means": means}):
         out, got = bsa_attention(q, k, v, shape, chunk_thw=chunk, top_k=top_k, return_indices=True, **kw, **more)
         assert torch.equal(got, idx) and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("D", [16, 32])
+def test_other_head_dims_match_stages(device, D):
+    q, k, v = _qkv(device, torch.float16, 2, 32, 32, D, seed=D)
+    shape, chunk = (1, 1, 2048), (1, 1, 64)
+    idx = select_block_indices(*(mean_pool_blocks_3d(t, shape, chunk) for t in (q, k)), 3)
+    out, got = bsa_attention(q, k, v, shape, chunk_thw=chunk, top_k=3, return_indices=True)
+    assert torch.equal(got, idx) and torch.equal(out, bsa_attention_hip(q, k, v, idx, chunk, shape))
 
 
 @pytest.mark.parametrize("H,nk", [(2, 319), (2, 320)])
