@@ -62,16 +62,6 @@ __device__ __forceinline__ void load8f(const float* p, float* v) {
   v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
 }
 
-template <typename T>
-__device__ __forceinline__ void widen8(const u32x4& raw, float* v) {
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const uint32_t w = raw[m];
-    v[2 * m] = to_f32(__builtin_bit_cast(T, (uint16_t)(w & 0xffffu)));
-    v[2 * m + 1] = to_f32(__builtin_bit_cast(T, (uint16_t)(w >> 16)));
-  }
-}
-
 // One wave per row; lane l holds the 8-element chunks l, l + 64, ... of the
 // row (NMAX chunks at most, so C <= 512 * NMAX).  HBM bound: all of a row's x and a
 // are loaded before the first use, and nothing in the kernel branches per lane

@@ -39,6 +39,17 @@ __device__ __forceinline__ float group_sum(float v) {
 // compiler would fold the FMA back into a plain multiply or add.
 __device__ __forceinline__ float mul1(float a, float b, float neg_zero) { return __builtin_fmaf(a, b, neg_zero); }
 
+// Eight T values to fp32.
+template <typename T>
+__device__ __forceinline__ void widen8(const u32x4& raw, float* v) {
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const uint32_t w = raw[m];
+    v[2 * m] = to_f32(__builtin_bit_cast(T, (uint16_t)(w & 0xffffu)));
+    v[2 * m + 1] = to_f32(__builtin_bit_cast(T, (uint16_t)(w >> 16)));
+  }
+}
+
 // Round an fp32 result to T in two steps, as the reference's fp32 op followed
 // by a cast does: the empty asm pins the fp32 value, so the compiler cannot
 // fold the conversion into the producing FMA (v_fma_mixlo_f16 rounds the

@@ -127,15 +127,6 @@ __device__ __forceinline__ u32x4 load_weight(const void* w, int c) {
   return u32x4{one | (one << 16), one | (one << 16), one | (one << 16), one | (one << 16)};
 }
 
-template <typename T>
-__device__ __forceinline__ void widen8(const u32x4& raw, float (&x)[8]) {
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    x[2 * m] = to_f32(__builtin_bit_cast(T, (uint16_t)(raw[m] & 0xffffu)));
-    x[2 * m + 1] = to_f32(__builtin_bit_cast(T, (uint16_t)(raw[m] >> 16)));
-  }
-}
-
 // RMSNorm of a row held 8 elements a lane over D / 8 lanes.
 template <typename T, int D>
 __device__ __forceinline__ void norm_row(const float (&x)[8], const u32x4& wr, float eps, float nz, float (&y)[8]) {

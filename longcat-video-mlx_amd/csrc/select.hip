@@ -747,7 +747,8 @@ hipError_t launch_select_tile(RouteArgs a, int BH, hipStream_t stream) {
 
 template <int NPER, int D>
 hipError_t launch_select_mfma_n(RouteArgs a, int BH, hipStream_t stream) {
-  if (select_short(BH, a.nq, a.nk, D)) return launch_select_tile<NPER, D, 8, 8>(a, BH, stream);
+  if constexpr (64 * NPER <= 256)  // select_short's rows
+    if (select_short(BH, a.nq, a.nk, D)) return launch_select_tile<NPER, D, 8, 8>(a, BH, stream);
   return launch_select_tile<NPER, D, 16, 4>(a, BH, stream);
 }
 
