@@ -35,6 +35,22 @@ def device():
     return torch.device("cuda", 0)
 
 
+@pytest.fixture
+def calls(monkeypatch):
+    """``calls(module, name)``: a list that grows with each call of that function."""
+    def watch(module, name):
+        seen, f = [], getattr(module, name)
+
+        def watched(*args, **kw):
+            seen.append(name)
+            return f(*args, **kw)
+
+        monkeypatch.setattr(module, name, watched)
+        return seen
+
+    return watch
+
+
 def assert_close_report(actual, expected, max_abs: float, mean_abs: float, what: str = ""):
     """max-abs / mean-abs parity check with a readable report."""
     import numpy as np

@@ -5,6 +5,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from lcv_bsa import dit_block
 from lcv_bsa.block_ops import adaln_modulation
 from lcv_bsa.dit_block import LongCatSingleStreamBlock
 
@@ -31,14 +32,16 @@ def test_matches_64_bits(device, dtype, K, B, T, C, chunks):
 
 
 @pytest.mark.parametrize("K", [64, 512, 36])
-def test_block_modulation_routes_agree(device, K):
+def test_block_modulation_routes_agree(device, calls, K):
     """Kernel and torch (K = 36 takes torch's on both sides)."""
+    kernel = calls(dit_block, "adaln_modulation")
     blk = LongCatSingleStreamBlock(256, 2, 4, K, dtype=torch.float16, device=device)
     t = torch.randn(2, 5, K, device=device)
     with torch.no_grad():
         for got, want in zip(blk._modulation(t, True), blk._modulation(t, False), strict=True):
             assert got.shape == want.shape == (2, 5, 1, 256) and got.dtype == torch.float32
             assert torch.allclose(got, want, rtol=1e-5, atol=2e-6)
+    assert len(kernel) == (K != 36)
 
 
 def test_a_weight_that_stands_for_others(device):

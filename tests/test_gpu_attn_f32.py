@@ -76,6 +76,7 @@ def test_error_no_larger_than_the_vector_alu(device, D, shape, chunk, kv_shape, 
     # exponent; the split adds below one more.  A quarter covers small samples.
     assert err <= 2e-6 and err <= 1.25 * err_valu, (float(err), float(err_valu))
     assert torch.equal(got, bsa_attention_hip(q, k, v, idx, **kw).double().cpu())
+    assert not torch.equal(got, valu)  # two kernels
 
 
 def test_strided_rows_negative_scale_and_skipped_entries(device):

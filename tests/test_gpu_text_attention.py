@@ -9,6 +9,7 @@ import pytest
 import torch
 from conftest import NORM_CHANGES, changed_norms
 
+from lcv_bsa import dit_block
 from lcv_bsa.block_ops import head_rms_norm, text_attention
 from lcv_bsa.block_sparse_attention import BSADeviceError
 from lcv_bsa.dit_block import MultiHeadCrossAttention, RMSNorm_FP32
@@ -132,24 +133,27 @@ def test_non_finite_values(device):
 
 @pytest.mark.parametrize("N", [100, 192])
 @pytest.mark.parametrize("text", [(50, 9), (64, 128)])
-def test_layer_routes_agree(device, N, text):
+def test_layer_routes_agree(device, calls, N, text):
     """The layer with the kernel, with torch's operations, and with a gradient
     wanted (which torch's operations give)."""
+    kernel = calls(dit_block, "text_attention")
     m = MultiHeadCrossAttention(256, 2, dtype=torch.float16, device=device)
     x = torch.randn(2, N, 256, device=device, dtype=torch.float16)
     y = torch.randn(1, sum(text), 256, device=device, dtype=torch.float16)
     with torch.no_grad():
         fused = m(x, y, text)
+        assert len(kernel) == 1
         m.fused = False
         plain = m(x, y, text)
         m.fused = True
+    assert len(kernel) == 1
     _check(fused, plain.float(), torch.float16)
     if N % 64 or any(n % 64 for n in text):
         x.requires_grad_()
         out = m(x, y, text)
         assert torch.equal(out, plain)
         out.sum().backward()
-        assert x.grad is not None
+        assert x.grad is not None and len(kernel) == 1
 
 
 @pytest.mark.parametrize("text", [(31, 33), (50, 9), (64, 128)])
