@@ -790,15 +790,16 @@ hipError_t launch_route(RouteArgs a, int BH, hipStream_t stream) {
 
 // One workgroup of 8 rows and 8 waves per CU at most, and one 32-key tile per
 // wave at most: routing is then one chain of loads, 48 MFMAs and a top-k, and one
-// launch instead of two.  Whole forward against scores + top-k, fp16: at D = 128 20.2 /
-// 22.3 us at 2 heads x 32 blocks, 30.9 / 33.0 at 8 x 64, 31.9 / 34.9 at 32 x 8 over 64,
-// 72.7 / 73.6 at 8 x 192, 37.8 / 37.5 at 8 x 1 over 192; at D = 64 48.0 / 50.4 at 16 x
-// 128, 51.4 / 53.5 at 12 x 160.  Beyond the line, D = 128: 121.1 / 121.4 at 8 x 256, 65.3 /
-// 64.3 at 32 x 8 over 256, 363 / 351 at 2 x 900, 114 / 106 at 32 x 100.  Other head dims
-// have no MFMA tiling of the fused kernel: 59.8 / 55.8 us at D = 32, 8 x 64 blocks, 41.8 /
-// 37.9 at D = 16, fp32, 2 x 64.
+// launch instead of two.  Whole forward against scores + top-k, fp16:
+//   D = 128: 20.2 / 22.3 us at 2 heads x 32 blocks, 30.9 / 33.0 at 8 x 64, 72.7 / 73.6
+//     at 8 x 192, 94.2 / 94.9 at 8 x 224, 49.3 / 49.2 at 2 x 224; few rows over more
+//     keys 31.9 / 34.9 at 32 x 8 over 64, 37.8 / 37.5 at 8 x 1 over 192;
+//   D = 64: 48.0 / 50.4 at 16 x 128, 51.4 / 53.5 at 12 x 160.
+// Beyond the line, D = 128: 121.1 / 121.4 at 8 x 256, 65.3 / 64.3 at 32 x 8 over 256,
+// 363 / 351 at 2 x 900, 114 / 106 at 32 x 100.  Other head dims have no MFMA tiling of
+// the fused kernel: 59.8 / 55.8 us at D = 32, 8 x 64, 41.8 / 37.9 at D = 16, fp32, 2 x 64.
 bool select_short(int BH, int nq, int nk, int D) {
-  return (D == 64 || D == 128) && nk <= 192 && (int64_t)BH * ((nq + 7) / 8) <= 256;
+  return (D == 64 || D == 128) && nk <= 224 && (int64_t)BH * ((nq + 7) / 8) <= 256;
 }
 
 bool select_supported(int nk, int D) {

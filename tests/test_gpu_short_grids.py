@@ -38,7 +38,7 @@ def _attend(q, k, v, idx, nq, nk, order):
 # 6,144 / 6,150 attention workgroups.
 GRIDS = [(1, 1, 1), (2, 32, 32), (2, 33, 33), (1, 256, 256), (1, 257, 257), (8, 256, 256), (9, 256, 256),
          (3, 7, 255), (1, 320, 320), (1, 321, 321), (2, 64, 321), (4, 1, 40),
-         (24, 256, 256), (25, 246, 246), (8, 192, 192), (2, 193, 193), (11, 190, 190), (8, 3, 192)]
+         (24, 256, 256), (25, 246, 246), (8, 224, 224), (2, 225, 225), (9, 224, 224), (10, 224, 224), (8, 3, 224)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
