@@ -15,13 +15,15 @@
 //
 // Measured against the vector-ALU kernel (attn_valu_kernel), which forms every
 // product from LDS operands: 8 heads x 12,480 tokens x 128, 13 of 195 blocks
-// kept (42.5 GFLOP), 1,763 -> 280 us (24 -> 152 TFLOP/s, what torch's fp32 GEMM
-// of 8192^3 reaches on this card is 153); 2 heads x 4,096 x 64, 4 of 64 kept:
-// 66.5 -> 15.6 us.  Error against 64 bits (2-norm) 6.9e-7 -> 4.7e-7 and
-// 4.0e-7 -> 2.7e-7.  At the first size the MFMA pipe is busy 39 % of the
-// cycles, the VALU (a third of it splitting K and V tiles) 32 %, LDS 29 %, with
-// no bank conflicts: what bounds it is how little the two or three workgroups of
-// a CU overlap these, and the last generation of workgroups.
+// kept (42.5 GFLOP), 1,763 -> 284 us (24 -> 150 TFLOP/s; torch's fp32 GEMM of
+// 8192^3 reaches 153 on this card); 2 heads x 4,096 x 64, 4 of 64 kept: 66.5 -> 16.2
+// us.  4 and 0.6 us of these are the check for small values and P's scaling, at D = 64
+// with longer lists (8 x 195 blocks) 5.7 of 164 us for the whole call.  Error against
+// 64 bits (2-norm) 6.9e-7 -> 4.7e-7 and 4.0e-7 -> 2.7e-7.  At the first size the MFMA
+// pipe is busy 39 % of the cycles, the VALU (a third of it splitting K and V tiles)
+// 32 %, LDS 29 %, with no bank conflicts (before the check): what bounds it is how
+// little the two or three workgroups of a CU overlap these, and the last generation
+// of workgroups.
 #include <algorithm>
 
 #include "attn_common.h"
@@ -127,9 +129,9 @@ __device__ __forceinline__ void slow_walk(const AttnParams& p, int bh, int qb, c
 }
 
 // Waves per SIMD.  D = 128 keeps 48 registers of Q pieces, 32 of O and up to 32
-// of tile prefetch: 180 in all, two waves (317 us at the first size above; held
-// to the 168 registers of three it spills Q pieces, 322).  D = 64 needs half of
-// each: four.
+// of tile prefetch: 196 in all, two waves (317 us for the whole call at the first
+// size above; held to the 168 registers of three it spills Q pieces, 322).  D = 64
+// needs half of each: four.
 template <int D>
 struct F32Occupancy {
   static constexpr int kWaves = D == 128 ? 2 : 4;

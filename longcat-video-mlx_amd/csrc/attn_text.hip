@@ -27,13 +27,14 @@
 // Work ids run batch item fastest: items of different text lengths share an
 // XCD's time, and each XCD's heads keep their text K / V in its L2.
 //
-// Measured at 28,800 queries x 32 heads x 128, bf16: 256 text tokens 150 to 165 us
-// (809 TFLOP/s at 150), 512 tokens 248 us (974 TFLOP/s), 13 tokens 81 us (5.8 TB/s);
-// two items of 231 and 13 tokens 301 us against 2,830 us for torch's norms,
-// copies and flash attention.  128-row workgroups against 64-row ones (twice the
-// tile fetches): 301 against 422 us.  Plain against non-temporal query loads:
-// 301 against 316 us.  Work ids by row tile with all heads together instead of
-// head by head: 320 against 316 us, and 332 against 265 us at 512 tokens.
+// Measured at 28,800 queries x 32 heads x 128, bf16, over the boxes seen: 256 text
+// tokens 150 to 190 us (809 TFLOP/s at 150), 512 tokens 248 to 272 us (974 TFLOP/s at
+// 248), 13 tokens 81 to 86 us (5.8 TB/s at 81); two items of 231 and 13 tokens 301 to 370
+// us against 2,830 us for torch's norms, copies and flash attention.  Against variants,
+// each on one box: 128-row workgroups against 64-row ones (twice the tile fetches) 301 /
+// 422 us; plain against non-temporal query loads 301 / 316 us; work ids head by head
+// against row tile by row tile with all heads together 316 / 320 us, and 265 / 332 us at
+// 512 tokens.  168 registers at D = 128, one spilled in bf16.
 #include "attn_common.h"
 #include "norm_common.h"
 
