@@ -344,7 +344,7 @@ class MultiHeadCrossAttention(nn.Module):
         if q.shape[1] % 64 == 0 and all(n % 64 == 0 for n in lens):
             return True
         n = lens[:q.shape[0]]
-        return (len(n) == q.shape[0] and min(n) >= 1 and sum(n) <= kv.shape[1]
+        return (q.numel() > 0 and len(n) == q.shape[0] and min(n) >= 1 and sum(n) <= kv.shape[1]
                 and plain_rms_norms(self.q_norm, self.k_norm)
                 and plain_tensors(q, kv, self.q_norm.weight, self.k_norm.weight)
                 and all(t.data_ptr() % 16 == 0 and t.stride(-1) == 1

@@ -202,6 +202,17 @@ def test_layer_runs_its_norms_as_modules(device, what):
         assert torch.equal(got, m(x, y, (50,)))
 
 
+@pytest.mark.parametrize("cond_only", [False, True])
+def test_layer_without_queries(device, cond_only):
+    """No token, or conditioning tokens alone, over ragged text."""
+    m = MultiHeadCrossAttention(256, 2, dtype=torch.float16, device=device)
+    x = torch.randn(2, 100 if cond_only else 0, 256, device=device, dtype=torch.float16)
+    y = torch.randn(1, 59, 256, device=device, dtype=torch.float16)
+    with torch.no_grad():
+        out = m(x, y, (50, 9), num_cond_latents=4 if cond_only else None, shape=(4, 5, 5) if cond_only else None)
+    assert out.shape == x.shape and (out == 0).all()
+
+
 def test_refused(device):
     q, kv, w = _inputs(device, torch.float16, (8, 8), 64, 2, 64, seed=1)
     k, v = kv[:, 0].transpose(0, 1), kv[:, 1].transpose(0, 1)
