@@ -408,7 +408,8 @@ class LongCatSingleStreamBlock(nn.Module):
         if (fused and t.dim() == 3 and t.is_cuda and w.device == b.device == t.device and unwatched(t, w, b)
                 and w.dtype == b.dtype and w.dtype in (torch.float16, torch.bfloat16)
                 and w.data_ptr() % 16 == 0 and w.is_contiguous() and w.shape[0] == 6 * self.hidden_size
-                and t.shape[-1] == w.shape[1] <= 1024 and w.shape[1] % 8 == 0
+                and 0 < t.shape[-1] == w.shape[1] <= 1024 and w.shape[1] % 8 == 0
+                and 0 < t.shape[0] * t.shape[1] <= 8 * 65535
                 and not torch.is_autocast_enabled("cuda")):
             tf = t.float()
             if tf.data_ptr() % 16 == 0:

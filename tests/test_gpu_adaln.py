@@ -60,3 +60,12 @@ def test_a_weight_that_stands_for_others(device):
             setattr(lin, name, doubled)
             for got, want in zip(blk._modulation(t, True), blk._modulation(t, False), strict=True):
                 assert torch.allclose(got, want, rtol=1e-5, atol=2e-6)
+
+
+@pytest.mark.parametrize("B,T,K", [(1, 8 * 65535 + 1, 8), (2, 0, 64), (0, 3, 64), (1, 2, 0)])
+def test_sizes_beyond_the_kernel_go_through_torch(device, B, T, K):
+    blk = LongCatSingleStreamBlock(8, 1, 4, K, dtype=torch.float16, device=device)
+    t = torch.randn(B, T, K, device=device)
+    with torch.no_grad():
+        for got, want in zip(blk._modulation(t, True), blk._modulation(t, False), strict=True):
+            assert got.shape == (B, T, 1, 8) and torch.equal(got, want)
